@@ -32,6 +32,21 @@ __device__ __forceinline__ bool cedge_keep(const PT& pd, uint32_t x) {
   return pd.bits ? (pd.bits[x >> 5] >> (x & 31u)) & 1u : (pd.mask[x] >> pd.bbit) & 1u;
 }
 
+// cedge_keep for neighbour x of v (degree dv), and in an oriented pair also
+// the order of the two: by degree, then id, x past v (orient 1) or before it
+// (orient 2).  The degree order keeps the lists of a power-law graph short:
+// the longest list towards higher degrees has 446 entries on the 2^20-vertex,
+// 8.75M-edge R-MAT graph, where ids leave half of the 42,300 neighbours.
+template <class PT>
+__device__ __forceinline__ bool cedge_keep(const PT& pd, const uint32_t* __restrict__ off, uint32_t v, uint32_t dv,
+                                           uint32_t x) {
+  if (!cedge_keep(pd, x)) return false;
+  if (!pd.orient) return true;
+  const uint32_t dx = off[x + 1] - off[x];
+  const bool past = dx != dv ? dx > dv : x > v;
+  return past == (pd.orient == 1);
+}
+
 // Pair of flat row f: the last pair whose first row is <= f.
 template <class PT>
 __device__ __forceinline__ uint32_t cedge_pair_index(const PT* __restrict__ P, uint32_t np, uint64_t f) {
@@ -151,7 +166,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_row_count(const PT* __restrict__
         x[t] = ok[t] ? adj[i] : 0u;
       }
 #pragma unroll
-      for (int t = 0; t < U; t++) ok[t] = ok[t] && cedge_keep(pd, x[t]);
+      for (int t = 0; t < U; t++) ok[t] = ok[t] && cedge_keep(pd, off, v, e - s, x[t]);
 #pragma unroll
       for (int t = 0; t < U; t++) got += (uint32_t)__popcll(__ballot(ok[t]) & gmask);
     }
@@ -192,7 +207,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_row_fill(const PT* __restrict__ 
         x[t] = ok[t] ? adj[i] : 0u;
       }
 #pragma unroll
-      for (int t = 0; t < U; t++) ok[t] = ok[t] && cedge_keep(pd, x[t]);
+      for (int t = 0; t < U; t++) ok[t] = ok[t] && cedge_keep(pd, off, v, e - s, x[t]);
 #pragma unroll
       for (int t = 0; t < U; t++) {
         const uint64_t bal = __ballot(ok[t]) & gmask;
@@ -220,6 +235,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_seg_cedge(const PT* __restrict__
                                                           const uint32_t* __restrict__ seg_row,
                                                           const uint32_t* __restrict__ seg_pair,
                                                           const uint2* __restrict__ seg_range,
+                                                          const uint32_t* __restrict__ off,
                                                           const uint32_t* __restrict__ adj,
                                                           uint32_t* __restrict__ segcnt,
                                                           unsigned long long* __restrict__ segbits,
@@ -237,6 +253,11 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_seg_cedge(const PT* __restrict__
     const uint2 range = seg_range[s];
     const uint32_t s0 = range.x, s1 = range.y;
     if (!FILL) {
+      uint32_t v = 0, dv = 0;
+      if (pd.orient) {
+        v = pd.acand[f - pd.flat];
+        dv = off[v + 1] - off[v];
+      }
       uint32_t x[8];
       bool ok[8];
 #pragma unroll
@@ -246,7 +267,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_seg_cedge(const PT* __restrict__
         x[t] = ok[t] ? adj[i] : 0u;
       }
 #pragma unroll
-      for (int t = 0; t < 8; t++) ok[t] = ok[t] && cedge_keep(pd, x[t]);
+      for (int t = 0; t < 8; t++) ok[t] = ok[t] && cedge_keep(pd, off, v, dv, x[t]);
       uint32_t got = 0;
       unsigned long long mine = 0;
 #pragma unroll
@@ -348,7 +369,7 @@ int seg_count(fsig_ctx* c, const PT* dP, uint32_t np, uint64_t rows, const uint3
   s_hi = std::min(s_hi, sr.nsegs);
   if (s_lo >= s_hi) return FSIG_OK;
   k_seg_cedge<PT, false><<<seg_grid(c, s_hi - s_lo), FSIG_BLOCK, 0, c->stream>>>(
-      dP, rows, sr.segbase, sr.seg_row, sr.seg_pair, sr.seg_range, adj, sr.segcnt, sr.segbits, cnt, nullptr, nullptr,
+      dP, rows, sr.segbase, sr.seg_row, sr.seg_pair, sr.seg_range, off, adj, sr.segcnt, sr.segbits, cnt, nullptr, nullptr,
       s_lo, s_hi);
   FSIG_HIP(c, hipGetLastError());
   return FSIG_OK;
@@ -360,7 +381,7 @@ int seg_fill(fsig_ctx* c, const PT* dP, uint32_t np, uint64_t rows, const uint32
   s_hi = std::min(s_hi, sr.nsegs);
   if (s_lo >= s_hi) return FSIG_OK;
   k_seg_cedge<PT, true><<<seg_grid(c, s_hi - s_lo), FSIG_BLOCK, 0, c->stream>>>(
-      dP, rows, sr.segbase, sr.seg_row, sr.seg_pair, sr.seg_range, adj, sr.segcnt, sr.segbits, nullptr, gscan,
+      dP, rows, sr.segbase, sr.seg_row, sr.seg_pair, sr.seg_range, off, adj, sr.segcnt, sr.segbits, nullptr, gscan,
       lst_all, s_lo, s_hi);
   FSIG_HIP(c, hipGetLastError());
   return FSIG_OK;

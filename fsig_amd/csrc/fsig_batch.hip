@@ -227,7 +227,8 @@ struct BPair {
   const uint32_t* bits;  // candidate bitmap of b (null: the mask)
   uint32_t* off_out;
   const uint32_t* bpos;  // vertex -> candidate index of b (null: binary search)
-  uint32_t asize, bsize, bbit, pad;
+  uint32_t asize, bsize, bbit;
+  uint32_t orient;  // 0: a batch counts without symmetry conditions
   uint64_t flat;
 };
 

@@ -406,8 +406,20 @@ static int match_impl(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
   uint64_t run_bound = max_emb;
   if (mode == FSIG_MODE_COUNT && !digest_out && c->tune.symmetry == 0 && plan_symmetry(P) && P.aut > 1 && max_emb)
     run_bound = max_emb / P.aut + (max_emb % P.aut != 0);
-  rc = alg == FSIG_ALG_MMATCH ? run_mmatch(c, g, P, mode, run_bound, count_out, emb_out, emb_cap, acc)
-                              : run_gsi(c, g, P, mode, run_bound, count_out, emb_out, emb_cap, acc);
+  if (alg == FSIG_ALG_MMATCH) {
+    bool by_degree = false;
+    for (uint32_t u = 0; u < k; u++) by_degree |= P.aut > 1 && P.sym_adj[u] != 0 && c->work_limit == 0;
+    const size_t mk2 = c->arena.mark(), timed = c->timed_used;
+    rc = run_mmatch(c, g, P, mode, run_bound, count_out, emb_out, emb_cap, acc, by_degree);
+    if (rc == FSIG_ENOMEM && by_degree) {
+      // the two orders build different tables: the arena may hold only the other's
+      c->arena.release(mk2);
+      c->timed_used = timed;
+      rc = run_mmatch(c, g, P, mode, run_bound, count_out, emb_out, emb_cap, acc, false);
+    }
+  } else {
+    rc = run_gsi(c, g, P, mode, run_bound, count_out, emb_out, emb_cap, acc);
+  }
   if (rc == FSIG_OK && P.aut > 1) {
     const uint64_t orbits = *count_out;
     *count_out = orbits > UINT64_MAX / P.aut ? UINT64_MAX : orbits * P.aut;

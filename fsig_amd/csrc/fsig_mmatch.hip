@@ -150,7 +150,8 @@ struct PairDesc {
   const uint32_t* bits;  // candidate bitmap of b (null: the mask)
   uint32_t* off_out;
   const uint32_t* bpos;  // vertex -> candidate index of b (null: binary search)
-  uint32_t asize, bsize, bbit, pad;
+  uint32_t asize, bsize, bbit;
+  uint32_t orient;  // 1 / 2: only neighbours past / before the candidate by degree (cedge_keep)
   uint64_t flat;  // first row of the pair in the flat row space
 };
 
@@ -172,12 +173,20 @@ struct MMatchProvider {
   const QueryPlan* P;
   const uint32_t* cand[MAXQ];  // per class
   uint32_t csize[MAXQ];
-  // pair lists: index by (class a, class b)
-  const uint32_t* poff[MAXQ][MAXQ];
-  const uint32_t* plst[MAXQ][MAXQ];
+  // pair lists: index by (orientation, class a, class b)
+  const uint32_t* poff[3][MAXQ][MAXQ];
+  const uint32_t* plst[3][MAXQ][MAXQ];
   // data vertex -> candidate index maps of the classes that have one (null:
   // binary search)
   const uint32_t* pos[MAXQ];
+  // symmetry conditions kept by oriented lists: adj_lt[u] has bit w when
+  // phi(u) comes before phi(w) by degree, for neighbours u and w
+  uint32_t adj_lt[MAXQ];
+
+  // orientation of the list that extends u's image by its neighbour w
+  uint32_t orient(uint32_t u, uint32_t w) const {
+    return ((adj_lt[u] >> w) & 1u) ? 1u : ((adj_lt[w] >> u) & 1u) ? 2u : 0u;
+  }
 
   JoinLevel level(uint32_t p) const {
     JoinLevel L;
@@ -191,6 +200,7 @@ struct MMatchProvider {
       const uint32_t u = P->order[c];
       if ((P->adjm[w] >> u) & 1u) {
         L.bcol[L.nb++] = c;
+        if (orient(u, w)) L.oriented = 1;
       } else if (P->label[u] == P->label[w]) {
         const uint32_t j = L.ncf++;
         L.cfcol[j] = c;
@@ -204,6 +214,7 @@ struct MMatchProvider {
     }
     for (uint32_t c = 0; c < p; c++) {  // symmetry conditions against earlier columns
       const uint32_t u = P->order[c];
+      if (orient(u, w)) continue;  // kept by the oriented list
       if ((P->sym_lt[u] >> w) & 1u) L.gtmask |= 1u << c;  // phi(u) < phi(w)
       if ((P->sym_lt[w] >> u) & 1u) L.ltmask |= 1u << c;  // phi(w) < phi(u)
     }
@@ -217,8 +228,8 @@ struct MMatchProvider {
     for (uint32_t c = 0; c < p; c++) {
       const uint32_t u = P->order[c];
       if ((P->adjm[w] >> u) & 1u) {
-        S.off[i] = poff[P->cls[u]][P->cls[w]];
-        S.lst[i] = plst[P->cls[u]][P->cls[w]];
+        S.off[i] = poff[orient(u, w)][P->cls[u]][P->cls[w]];
+        S.lst[i] = plst[orient(u, w)][P->cls[u]][P->cls[w]];
         i++;
       }
     }
@@ -241,7 +252,7 @@ static uint32_t refine_lanes(const fsig_graph* g) {
 }
 
 int run_mmatch(fsig_ctx* c, const fsig_graph* g, QueryPlan& P, int mode, uint64_t max_emb, uint64_t* count_out,
-               uint32_t* emb_out, uint64_t emb_cap, unsigned long long* digest_acc) {
+               uint32_t* emb_out, uint64_t emb_cap, unsigned long long* digest_acc, bool by_degree) {
   const uint32_t nc = P.nclass, k = P.k;
   Arena& A = c->arena;
   int rc;
@@ -391,58 +402,61 @@ int run_mmatch(fsig_ctx* c, const fsig_graph* g, QueryPlan& P, int mode, uint64_
 
   // ---- join order and the class pairs it needs
   plan_order_mmatch(P, size);
-  std::vector<PairDesc> pairs;
-  int pair_id[MAXQ][MAXQ];
-  for (auto& row : pair_id) for (int& x : row) x = -1;
-  for (uint32_t p = 1; p < k; p++) {
-    const uint32_t w = P.order[p];
-    for (uint32_t cpos = 0; cpos < p; cpos++) {
-      const uint32_t u = P.order[cpos];
-      if (!((P.adjm[w] >> u) & 1u)) continue;
-      const uint32_t a = P.cls[u], b = P.cls[w];
-      if (pair_id[a][b] >= 0) continue;
-      pair_id[a][b] = (int)pairs.size();
-      PairDesc pd;
-      pd.bpos = nullptr;
-      pd.acand = cur[a];
-      pd.bcand = cur[b];
-      pd.asize = size[a];
-      pd.bsize = size[b];
-      pd.bbit = b;
-      pd.mask = mask;
-      pd.bits = nullptr;
-      pd.off_out = nullptr;
-      pd.pad = 0;
-      pd.flat = 0;
-      pairs.push_back(pd);
-    }
-  }
   MMatchProvider pv;
   std::memset(&pv, 0, sizeof(pv));
   pv.P = &P;
   pv.chain_p = 0xffffffffu;
   for (uint32_t a = 0; a < nc; a++) { pv.cand[a] = cur[a]; pv.csize[a] = size[a]; }
+  // Symmetry conditions between neighbours go by degree and into the lists:
+  // 0.67e9 entries to intersect instead of 0.99e9 for the triangle on the
+  // 2^20-vertex R-MAT graph, and none of them in a hub's list
+  // (the sense of each step so that most of its lists run towards higher
+  // degrees).  Not under a work limit: the rows of a search that the limit
+  // counts would be others.
+  if (by_degree)
+    for (uint32_t v = 0; v < k; v++) {
+      uint32_t after = 0;
+      for (uint32_t m = P.sym_adj[v]; m; m &= m - 1) after += P.pos[__builtin_ctz(m)] > P.pos[v];
+      const bool first = 2 * after >= (uint32_t)__builtin_popcount(P.sym_adj[v]);
+      for (uint32_t m = P.sym_adj[v]; m; m &= m - 1) {
+        const uint32_t w = __builtin_ctz(m);
+        if (first) pv.adj_lt[v] |= 1u << w;
+        else pv.adj_lt[w] |= 1u << v;
+      }
+    }
+  std::vector<PairDesc> pairs;
+  int pair_id[3][MAXQ][MAXQ];
+  for (auto& t : pair_id) for (auto& row : t) for (int& x : row) x = -1;
+  auto add_pair = [&](uint32_t o, uint32_t a, uint32_t b) {
+    if (pair_id[o][a][b] >= 0) return;
+    pair_id[o][a][b] = (int)pairs.size();
+    PairDesc pd;
+    pd.bpos = nullptr;
+    pd.acand = cur[a];
+    pd.bcand = cur[b];
+    pd.asize = size[a];
+    pd.bsize = size[b];
+    pd.bbit = b;
+    pd.orient = o;
+    pd.mask = mask;
+    pd.bits = nullptr;
+    pd.off_out = nullptr;
+    pd.flat = 0;
+    pairs.push_back(pd);
+  };
+  for (uint32_t p = 1; p < k; p++) {
+    const uint32_t w = P.order[p];
+    for (uint32_t cpos = 0; cpos < p; cpos++) {
+      const uint32_t u = P.order[cpos];
+      if ((P.adjm[w] >> u) & 1u) add_pair(pv.orient(u, w), P.cls[u], P.cls[w]);
+    }
+  }
   // A count whose last two levels form a chain (see ChainTail) also needs
   // the reverse pair (last class -> previous class).
   const bool chain = mode == FSIG_MODE_COUNT && k >= 3 && c->tune.fused_tail == 0 &&
                      chain_tail_applies(pv.level(k - 2), pv.level(k - 1));
   const uint32_t cls_w = P.cls[P.order[k - 1]], cls_p = P.cls[P.order[k >= 2 ? k - 2 : 0]];
-  if (chain && pair_id[cls_w][cls_p] < 0) {
-    pair_id[cls_w][cls_p] = (int)pairs.size();
-    PairDesc pd;
-    pd.bpos = nullptr;
-    pd.acand = cur[cls_w];
-    pd.bcand = cur[cls_p];
-    pd.asize = size[cls_w];
-    pd.bsize = size[cls_p];
-    pd.bbit = cls_p;
-    pd.mask = mask;
-    pd.bits = nullptr;
-    pd.off_out = nullptr;
-    pd.pad = 0;
-    pd.flat = 0;
-    pairs.push_back(pd);
-  }
+  if (chain) add_pair(0, cls_w, cls_p);
   double avg_list = 1;
   if (!pairs.empty()) {
     KTimer tc(c, FSIG_K_CEDGE);
@@ -512,13 +526,13 @@ int run_mmatch(fsig_ctx* c, const fsig_graph* g, QueryPlan& P, int mode, uint64_
     std::vector<uint64_t> hb(np);
     for (uint32_t i = 0; i < np; i += 4096)
       if ((rc = read_u64(c, pbase + i, hb.data() + i, std::min<uint32_t>(4096, np - i)))) return rc;
-    for (uint32_t a = 0; a < nc; a++)
-      for (uint32_t b = 0; b < nc; b++)
-        if (pair_id[a][b] >= 0) {
-          const PairDesc& pd = pairs[pair_id[a][b]];
-          pv.poff[a][b] = pd.off_out;
-          pv.plst[a][b] = lst_all + hb[pair_id[a][b]];
-        }
+    for (uint32_t o = 0; o < 3; o++)
+      for (uint32_t a = 0; a < nc; a++)
+        for (uint32_t b = 0; b < nc; b++)
+          if (pair_id[o][a][b] >= 0) {
+            pv.poff[o][a][b] = pairs[pair_id[o][a][b]].off_out;
+            pv.plst[o][a][b] = lst_all + hb[pair_id[o][a][b]];
+          }
     avg_list = flat ? (double)total_edges / (double)flat : 1;
     // bytes: both passes read each row's candidate and offsets and, per
     // adjacency entry, the entry and its mask word; the fill reads the
@@ -535,10 +549,10 @@ int run_mmatch(fsig_ctx* c, const fsig_graph* g, QueryPlan& P, int mode, uint64_
     if (!sum) return set_err(c, FSIG_ENOMEM, "join: arena exhausted for the chain tail");
     KTimer tt(c, FSIG_K_JOIN_TAIL);
     k_chain_sum<16><<<grid_for(c, nv, FSIG_BLOCK / 16), FSIG_BLOCK, 0, c->stream>>>(
-        pv.poff[cls_c1][cls_p], pv.plst[cls_c1][cls_p], pv.poff[cls_p][cls_w], nv, sum);
+        pv.poff[0][cls_c1][cls_p], pv.plst[0][cls_c1][cls_p], pv.poff[0][cls_p][cls_w], nv, sum);
     FSIG_HIP(c, hipGetLastError());
     tt.done(16ull * nv, 0);  // offsets of each list; its entries and own offsets are charged by the tail
-    pv.chain = ChainTail{sum, pv.poff[cls_w][cls_p], pv.plst[cls_w][cls_p]};
+    pv.chain = ChainTail{sum, pv.poff[0][cls_w][cls_p], pv.plst[0][cls_w][cls_p]};
     pv.chain_p = k - 2;
   }
 

@@ -148,6 +148,9 @@ struct QueryPlan {
   // the count is aut times the number of embeddings that satisfy all of them
   uint64_t aut = 1;
   uint32_t sym_lt[MAXQ] = {0};
+  // the conditions of sym_lt whose stabiliser step asks them of neighbours
+  // only: any total order may stand for < in such a step
+  uint32_t sym_adj[MAXQ] = {0};
 };
 
 int plan_classes(QueryPlan& P, uint32_t k, const int32_t* qlabels, const uint32_t* qoff,
@@ -219,7 +222,10 @@ int read_u64(fsig_ctx* c, const void* dev, uint64_t* host, size_t count);
 // digest_acc (two zeroed device words, may be null): enumerate every
 // embedding and fold it into the order-independent set digest there instead
 // of copying rows to emb_out.
+// by_degree: symmetry conditions between neighbours (P.sym_adj) order them by
+// degree instead of id.
 int run_mmatch(fsig_ctx* c, const fsig_graph* g, QueryPlan& P, int mode, uint64_t max_emb,
-               uint64_t* count_out, uint32_t* emb_out, uint64_t emb_cap, unsigned long long* digest_acc);
+               uint64_t* count_out, uint32_t* emb_out, uint64_t emb_cap, unsigned long long* digest_acc,
+               bool by_degree);
 int run_gsi(fsig_ctx* c, const fsig_graph* g, QueryPlan& P, int mode, uint64_t max_emb,
             uint64_t* count_out, uint32_t* emb_out, uint64_t emb_cap, unsigned long long* digest_acc);

@@ -49,7 +49,9 @@ struct JoinLevel {
   // every column in gtmask and stay below that of every column in ltmask
   // (columns of w's class: the words compare as the data vertex ids do)
   uint32_t gtmask, ltmask;
+  uint32_t oriented;  // some list keeps a symmetry condition itself (ordered by degree)
 };
+
 
 constexpr uint32_t kNone = 0xffffffffu;
 
@@ -343,7 +345,9 @@ struct TailLds {
   uint32_t* s2;
   uint32_t* n2;
   uint32_t* cf2;
-  uint32_t* slot;  // G words: children counted by the group
+  uint32_t* slot;  // G words each: children counted by the group, and the
+  uint32_t* cs;    // starts and the scanned lengths of their own lists
+  uint32_t* pre;
   uint32_t* tile;  // tw words
   uint32_t tw;
 };
@@ -354,19 +358,26 @@ __device__ __forceinline__ void lds_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Lists of the leaf level: only shared ones (of parent columns), only the
+// child's own, or both.
+enum TailKind : int { kTailAny = -1, kTailShared = 0, kTailOwn = 1, kTailBoth = 2 };
+
 // Leaves of one parent row; returns this lane's share of the leaf count
 // (sum over the group's lanes = the row's leaves) and sets `children` (group
-// uniform) to the number of children x.
-template <int G>
+// uniform) to the number of children x.  KIND: the leaf level's lists, where
+// the launch knows them (the other kinds' registers are then not held).
+// kids_are_shared (kTailBoth, see tail_kids_shared): the children are I.
+template <int G, int KIND = kTailAny>
 __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdgeSrc& S1, const JoinLevel& L2,
                                              const CandEdgeSrc& S2, const uint32_t (&rv)[(MAXQ + G - 1) / G],
                                              const TailLds& sh, uint32_t gl, uint64_t gmask, uint64_t below,
-                                             uint64_t& children, bool& defer, unsigned long long& bytes) {
+                                             uint64_t& children, bool& defer, unsigned long long& bytes,
+                                             bool kids_are_shared = false) {
   const uint32_t p = L1.p;
   defer = false;
   uint32_t dlen = L1.wsize, d = 0;
   uint64_t el = 0;
-  for (uint32_t i = 0; i < L1.nb; i++) {
+  for (uint32_t i = 0; i < L1.nb && !kids_are_shared; i++) {
     const uint32_t x = group_col<G>(rv, L1.bcol[i]);
     const uint32_t s = S1.off[i][x], n = S1.off[i][x + 1] - s;
     sh.s1[i] = s;
@@ -404,7 +415,7 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
     sh.cf2[j] = t;
   }
   uint64_t lbytes = gl == 0 ? 4ull * p + 8ull * (L1.nb + ns) + 4ull * el : 0;
-  const uint32_t* dl = L1.nb ? S1.lst[d] + sh.s1[d] : nullptr;
+  const uint32_t* dl = L1.nb && !kids_are_shared ? S1.lst[d] + sh.s1[d] : nullptr;
   // symmetry conditions: children x in [lo1, hi1) (driver positions [ta1,
   // tb1)); leaves y in [lo2, hi2), and above (g2p) or below (l2p) their own
   // x
@@ -417,7 +428,7 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
   }
   if ((L2.gtmask | L2.ltmask) & ~pbit) sym_bounds<G>(L2.gtmask & ~pbit, L2.ltmask & ~pbit, rv, lo2, hi2);
   const bool leaf_bounds = lo2 != 0 || hi2 != kNone;
-  if (own == kNone) {
+  if (KIND == kTailShared || (KIND == kTailAny && own == kNone)) {
     // No own list: every child has the same leaves I except its own image.
     // |I| once per parent (one shared list: its length minus the conflicts
     // found in it; more: a counting walk), then one membership test per child.
@@ -503,12 +514,12 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
   // A row whose shared intersection does not fit the tile, or that may have
   // very many children (> 16G) while I is large (> 4G), is deferred: its
   // children are counted here and written by the caller, which counts their
-  // leaves one row per group.  Other rows stage I in LDS once and count each
-  // child's leaves cooperatively: lanes split the shorter of I and the
-  // child's own list and search the other.
+  // leaves one row per group.  Other rows stage I in LDS once and count the
+  // leaves of G children at a time.
   bool defer_row = false;
   uint32_t isz = 0;
-  if (ns > 0) {
+  const bool both = KIND == kTailBoth || (KIND == kTailAny && ns > 0);
+  if (both) {
     const uint32_t* dl2 = S2.lst[ds] + sh.s2[ds];
     uint32_t a2 = 0, b2 = dslen;
     if (leaf_bounds) driver_window(dl2, nullptr, false, dslen, lo2, hi2, a2, b2);
@@ -523,21 +534,56 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
       for (uint32_t j = 0; j < L2.ncf && ok; j++) ok = y != sh.cf2[j];
       const uint64_t bal = __ballot(ok) & gmask;
       const uint32_t nb = (uint32_t)__popcll(bal);
-      if (isz + nb > sh.tw) { defer_row = true; break; }  // I does not fit
-      if (ok) sh.tile[isz + __popcll(bal & below)] = y;
+      if (isz + nb > sh.tw) {  // I does not fit
+        defer_row = true;
+        if (!kids_are_shared) break;
+      }
+      if (ok && !defer_row) sh.tile[isz + __popcll(bal & below)] = y;
       isz += nb;
     }
     lds_wave_sync();
     // many children, each with a large I to intersect: spread them instead
+    if (kids_are_shared) tb1 = isz;
     defer_row = defer_row || (tb1 - ta1 > 16u * G && isz > 4u * G);
+    if (defer_row && kids_are_shared) {
+      defer = true;
+      children = isz;
+      bytes += lbytes;
+      return 0;
+    }
+  }
+  // I as an open-addressing hash set behind its list in the tile, a quarter
+  // to half full, when several children will be intersected with it: a child's
+  // list is then read through once, in coalesced steps, and each entry costs
+  // about two LDS reads instead of a chain of dependent gathers.  Bound by
+  // the latency of those reads and of the row's own range lookups.  With
+  // lists ordered by degree, the triangle on the 2^20-vertex, 8.75M-edge
+  // R-MAT graph went from 27.7 to 7.1 ms and the 4-clique on the 2^18-vertex,
+  // 2.19M-edge one from 37.6 to 8.0 ms (one child at a time and binary
+  // searches, ordered by degree: 17.5 and 11.8 ms).
+  uint32_t hsize = 0, hshift = 0;
+  uint32_t* hset = sh.tile + isz;
+  if (both && !defer_row && 2 * isz > (uint32_t)G && tb1 - ta1 > 2) {
+    hshift = __builtin_clz(2 * isz - 1) - 1;
+    if (isz + (1u << (32 - hshift)) > sh.tw) hshift++;
+    hsize = 1u << (32 - hshift);
+    if (isz + hsize > sh.tw) hsize = 0;
+    for (uint32_t e = gl; e < hsize; e += G) hset[e] = kNone;
+    lds_wave_sync();
+    for (uint32_t e = gl; e < isz && hsize; e += G) {
+      const uint32_t y = sh.tile[e];
+      uint32_t h = (y * 0x9e3779b1u) >> hshift;
+      while (atomicCAS(&hset[h], kNone, y) != kNone) h = (h + 1) & (hsize - 1);
+    }
+    lds_wave_sync();
   }
   uint64_t kids = 0, leaves = 0;
   for (uint32_t t0 = ta1; t0 < tb1; t0 += G) {
     const uint32_t t = t0 + gl;
     bool ok = t < tb1;
     uint32_t x = 0;
-    if (ok) x = L1.nb ? dl[t] : t;
-    for (uint32_t i = 0; i < L1.nb && ok; i++) {
+    if (ok) x = kids_are_shared ? sh.tile[t] : L1.nb ? dl[t] : t;
+    for (uint32_t i = 0; i < L1.nb && ok && !kids_are_shared; i++) {
       if (i == d) continue;
       ok = sorted_contains(S1.lst[i] + sh.s1[i], sh.n1[i], x);
     }
@@ -548,7 +594,7 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
     const uint64_t bal = __ballot(ok) & gmask;
     kids += __popcll(bal);
     if (defer_row) continue;
-    if (ns == 0) {
+    if (!both) {
       // own list only: its length minus the parent-column conflicts in it
       if (ok) {
         const uint32_t s = S2.off[own][x], n = S2.off[own][x + 1] - s;
@@ -565,32 +611,95 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
       }
       continue;
     }
+    const uint32_t nsurv = (uint32_t)__popcll(bal);
+    if (isz == 0 || nsurv == 0) continue;
+    // The surviving children of this step, one per lane: their own lists,
+    // laid end to end by an exclusive scan of the lengths.
     if (ok) sh.slot[__popcll(bal & below)] = x;
     lds_wave_sync();
-    const uint32_t nsurv = (uint32_t)__popcll(bal);
-    for (uint32_t q = 0; q < nsurv; q++) {
-      const uint32_t xx = sh.slot[q];
-      const uint32_t s = S2.off[own][xx], n = S2.off[own][xx + 1] - s;
-      const uint32_t* l = S2.lst[own] + s;
-      // leaves above (g2p) or below (l2p) the child itself
-      const uint32_t lox = g2p ? xx + 1 : 0, hix = l2p ? xx : kNone;
-      uint32_t got = 0;
-      if (isz <= n) {
-        for (uint32_t e0 = 0; e0 < isz; e0 += G) {
-          const uint32_t e = e0 + gl;
-          const bool in = e < isz && sh.tile[e] >= lox && sh.tile[e] < hix && sorted_contains(l, n, sh.tile[e]);
-          got += (uint32_t)__popcll(__ballot(in) & gmask);
+    uint32_t cs = 0, cn = 0;
+    if (gl < nsurv) {
+      const uint32_t xx = sh.slot[gl];
+      cs = S2.off[own][xx];
+      cn = S2.off[own][xx + 1] - cs;
+    }
+    uint32_t pre = cn;
+#pragma unroll
+    for (int o = 1; o < G; o <<= 1) {
+      const uint32_t t2 = __shfl_up(pre, o, G);
+      if (gl >= (uint32_t)o) pre += t2;
+    }
+    const uint32_t tot = __shfl(pre, G - 1, G);
+    sh.cs[gl] = cs;
+    sh.pre[gl] = pre - cn;
+    lds_wave_sync();
+    const uint32_t* ol = S2.lst[own];
+    const uint32_t pairs = nsurv * isz, lg = 32 - __builtin_clz((tot / nsurv) | 1);
+    if (gl == 0) lbytes += 8ull * nsurv;
+    if ((uint64_t)tot * (hsize ? 1 : 32 - __builtin_clz(isz)) <= (uint64_t)pairs * lg) {
+      // read the lists through: sub-groups of 8 lanes take every (G/8)th
+      // child, four strides of its list in flight, each entry looked up in I
+      constexpr uint32_t SG = G < 8 ? G : 8, NS = G / SG;
+      const uint32_t sl = gl & (SG - 1);
+      uint32_t j = gl / SG, at = 0, n = 0, xx = 0;
+      const uint32_t* l = ol;
+      bool open = false;  // child j is being read: entries [at, n) of l are left
+      for (;;) {
+        if (!open && j < nsurv) {
+          l = ol + sh.cs[j];
+          n = (j + 1 < (uint32_t)G ? sh.pre[j + 1] : tot) - sh.pre[j];
+          xx = sh.slot[j];
+          at = 0;
+          open = true;
         }
-        if (gl == 0) lbytes += 8 + 4ull * isz * (32 - __builtin_clz(n | 1));
-      } else {
-        for (uint32_t e0 = 0; e0 < n; e0 += G) {
-          const uint32_t e = e0 + gl;
-          const bool in = e < n && l[e] >= lox && l[e] < hix && sorted_contains(sh.tile, isz, l[e]);
-          got += (uint32_t)__popcll(__ballot(in) & gmask);
+        if (!open) break;
+        uint32_t y[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const uint32_t e = at + u * SG + sl;
+          y[u] = e < n ? l[e] : kNone;
         }
-        if (gl == 0) lbytes += 8 + 4ull * n;
+        at += 4 * SG;
+        if (at >= n) { open = false; j += NS; }
+        if (g2p | l2p) {  // leaves above (g2p) or below (l2p) the child itself
+#pragma unroll
+          for (int u = 0; u < 4; u++)
+            if ((g2p && y[u] <= xx) || (l2p && y[u] >= xx)) y[u] = kNone;
+        }
+        if (hsize) {
+          uint32_t h[4];
+#pragma unroll
+          for (int u = 0; u < 4; u++) h[u] = (y[u] * 0x9e3779b1u) >> hshift;
+          bool more;
+          do {  // the four chains advance together
+            uint32_t v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = hset[h[u]];
+            more = false;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+              leaves += v[u] == y[u] && y[u] != kNone;
+              const bool on = v[u] != y[u] && v[u] != kNone && y[u] != kNone;
+              h[u] = (h[u] + 1) & (hsize - 1);
+              if (!on) y[u] = kNone;
+              more |= on;
+            }
+          } while (more);
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; u++) leaves += y[u] != kNone && sorted_contains(sh.tile, isz, y[u]);
+        }
       }
-      if (gl == 0) leaves += got;
+      if (gl == 0) lbytes += 4ull * tot;
+    } else {
+      // search them: one (child, entry of I) pair per lane and step
+      for (uint32_t e = gl; e < pairs; e += G) {
+        const uint32_t j = e / isz;
+        const uint32_t y = sh.tile[e - j * isz], xx = sh.slot[j];
+        const uint32_t s = sh.cs[j], n = (j + 1 < (uint32_t)G ? sh.pre[j + 1] : tot) - sh.pre[j];
+        leaves += !(g2p && y <= xx) && !(l2p && y >= xx) && sorted_contains(ol + s, n, y);
+      }
+      if (gl == 0) lbytes += 4ull * pairs * lg;
     }
     lds_wave_sync();
   }
@@ -620,9 +729,9 @@ struct TailShared {
   static constexpr uint32_t kTileWords = 4096 / GPB;  // at most 16 KiB of tiles per block
   uint32_t s1[GPB][N1], n1[GPB][N1], cf1[GPB][N1];
   uint32_t s2[GPB][N2], n2[GPB][N2], cf2[GPB][N2];
-  uint32_t slot[GPB][G];
+  uint32_t slot[GPB][G], cs[GPB][G], pre[GPB][G];
   __device__ TailLds at(uint32_t gw, uint32_t* tile, uint32_t tw) {
-    return TailLds{s1[gw], n1[gw], cf1[gw], s2[gw], n2[gw], cf2[gw], slot[gw], tile + gw * tw, tw};
+    return TailLds{s1[gw], n1[gw], cf1[gw], s2[gw], n2[gw], cf2[gw], slot[gw], cs[gw], pre[gw], tile + gw * tw, tw};
   }
 };
 
@@ -633,15 +742,16 @@ struct TailIO {
   unsigned long long* res;    // [0] += leaves, [1] += children of counted rows
   unsigned long long* stats;  // [0] += algorithmic bytes, [1] += parent rows
   uint32_t tile_words;        // shared-intersection tile per group (dynamic LDS)
+  uint32_t kids_are_shared;   // the child level intersects the leaf's shared lists
 };
 
 // N: entries of the per-group list and conflict arrays of both levels.  At
 // most 72 VGPRs, so seven waves per SIMD fit where LDS allows (the tail is
 // bound by dependent gathers; eight waves need spills and run slower); 64
 // four-lane groups with 16-entry arrays fit six per SIMD by their LDS.
-template <int G, int N>
+template <int G, int N, int KIND>
 __global__ void __launch_bounds__(FSIG_BLOCK)
-    __attribute__((amdgpu_waves_per_eu(G == 4 && N > (int)kTailSmall ? 6 : 7, 8)))
+    __attribute__((amdgpu_waves_per_eu(G == 4 && N > (int)kTailSmall ? 5 : 7, 8)))
 k_join_tail(JoinLevel L1, CandEdgeSrc S1, JoinLevel L2, CandEdgeSrc S2, TailIO io) {
   constexpr int GPB = FSIG_BLOCK / G;
   constexpr int NR = (MAXQ + G - 1) / G;
@@ -663,7 +773,8 @@ k_join_tail(JoinLevel L1, CandEdgeSrc S1, JoinLevel L2, CandEdgeSrc S2, TailIO i
     }
     uint64_t kids = 0;
     bool defer = false;
-    my_leaves += tail_row<G>(L1, S1, L2, S2, rv, t, gl, gmask, below, kids, defer, my_bytes);
+    my_leaves += tail_row<G, KIND>(L1, S1, L2, S2, rv, t, gl, gmask, below, kids, defer, my_bytes,
+                                  KIND == kTailBoth && io.kids_are_shared);
     if (gl == 0) {
       io.cnt[r] = defer ? (uint32_t)kids : 0u;
       if (!defer) my_kids += kids;
@@ -698,13 +809,30 @@ inline bool tail_applies(const JoinLevel& L2) {
   return false;
 }
 
+// Whether the children of level L1 are the shared intersection of the leaf
+// level L2 itself (the last two vertices of a clique): the same lists of the
+// same columns, and no conflict or bound on either.
+inline bool tail_kids_shared(const JoinLevel& L1, const CandEdgeSrc& S1, const JoinLevel& L2, const CandEdgeSrc& S2) {
+  if (L2.nb != L1.nb + 1 || L1.nb == 0 || L1.ncf || L2.ncf) return false;
+  if (L1.gtmask | L1.ltmask | L2.gtmask | L2.ltmask) return false;
+  uint32_t j = 0;  // both list their columns in ascending order
+  for (uint32_t i = 0; i < L2.nb; i++) {
+    if (L2.bcol[i] == L1.p) continue;
+    if (j >= L1.nb || L1.bcol[j] != L2.bcol[i] || S1.off[j] != S2.off[i] || S1.lst[j] != S2.lst[i]) return false;
+    j++;
+  }
+  return j == L1.nb;
+}
+
 // Tile words per group the tail of L2 needs: only a leaf with both shared
 // lists (parent columns) and an own list (column p) intersects in LDS.
+// 16 KiB per block; twice that where lists ordered by degree are intersected,
+// whose few hundred entries then fit beside their hash set.
 inline uint32_t tail_tile_words(uint32_t G, const JoinLevel& L2, uint32_t cap) {
   bool shared = false, own = false;
   for (uint32_t i = 0; i < L2.nb; i++) (L2.bcol[i] == L2.p - 1 ? own : shared) = true;
   if (!shared || !own) return 0;
-  const uint32_t w = 4096 / (FSIG_BLOCK / G);
+  const uint32_t w = (L2.oriented ? 8192 : 4096) / (FSIG_BLOCK / G);
   return cap && cap < w ? cap : w;
 }
 
@@ -717,9 +845,14 @@ inline int launch_join_tail(fsig_ctx* c, uint32_t G, const JoinLevel& L1, const 
   const uint32_t grid = (uint32_t)std::max<uint64_t>(blocks, 1);
   const size_t lds = (size_t)io.tile_words * gpb * sizeof(uint32_t);
   const bool small = L1.nb <= kTailSmall && L1.ncf <= kTailSmall && L2.nb <= kTailSmall && L2.ncf <= kTailSmall;
-#define FSIG_TAIL(GV)                                                                       \
-  (small ? k_join_tail<GV, kTailSmall><<<grid, FSIG_BLOCK, lds, c->stream>>>(L1, S1, L2, S2, io) \
-         : k_join_tail<GV, kTailMax><<<grid, FSIG_BLOCK, lds, c->stream>>>(L1, S1, L2, S2, io))
+  bool shared = false, own = false;
+  for (uint32_t i = 0; i < L2.nb; i++) (L2.bcol[i] == L1.p ? own : shared) = true;
+#define FSIG_TAIL_N(GV, KV)                                                                      \
+  (small ? k_join_tail<GV, kTailSmall, KV><<<grid, FSIG_BLOCK, lds, c->stream>>>(L1, S1, L2, S2, io) \
+         : k_join_tail<GV, kTailMax, KV><<<grid, FSIG_BLOCK, lds, c->stream>>>(L1, S1, L2, S2, io))
+#define FSIG_TAIL(GV)                                                                  \
+  (shared && own ? FSIG_TAIL_N(GV, kTailBoth) : own ? FSIG_TAIL_N(GV, kTailOwn) \
+                                                    : FSIG_TAIL_N(GV, kTailShared))
   switch (G) {
     case 4: FSIG_TAIL(4); break;
     case 8: FSIG_TAIL(8); break;
@@ -728,6 +861,7 @@ inline int launch_join_tail(fsig_ctx* c, uint32_t G, const JoinLevel& L1, const 
     default: FSIG_TAIL(64); break;
   }
 #undef FSIG_TAIL
+#undef FSIG_TAIL_N
   FSIG_HIP(c, hipGetLastError());
   return FSIG_OK;
 }
@@ -889,7 +1023,8 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_join_tail_chain(JoinLevel L1, Ca
 // Whether the chain tail applies to levels p (L1) and p+1 (L2).
 inline bool chain_tail_applies(const JoinLevel& L1, const JoinLevel& L2) {
   return L2.nb == 1 && L2.bcol[0] == L1.p && L1.nb == 1 && L1.ncf <= kTailMax && L2.ncf <= kTailMax &&
-         !(L1.gtmask | L1.ltmask | L2.gtmask | L2.ltmask);  // its sums cover every child and leaf
+         !(L1.gtmask | L1.ltmask | L2.gtmask | L2.ltmask) &&  // its sums cover every child and leaf
+         !L1.oriented && !L2.oriented;                        // and its reverse lists are whole
 }
 
 inline int launch_join_tail_chain(fsig_ctx* c, uint32_t G, const JoinLevel& L1, const CandEdgeSrc& S1,
@@ -1154,11 +1289,14 @@ class JoinDriver {
     // through the LDS tile, else few (rows are mostly a handful of dependent
     // gathers: more of them in flight)
     const bool needs_tile = tail_tile_words(8, L2, 0) != 0;
-    const uint32_t G = widen_lanes(c_, use_chain || !needs_tile ? std::min<uint32_t>(std::max<uint32_t>(G_, 4), 8)
-                                                                : std::max<uint32_t>(G_, 8),
-                                   R, use_chain ? 32 : 64);
+    // (64 for lists ordered by degree: the widest tile, which holds all of
+    // them with their hash sets)
+    const uint32_t G0 = use_chain || !needs_tile ? std::min<uint32_t>(std::max<uint32_t>(G_, 4), 8)
+                        : L2.oriented && L2.nb == 2 && !c_->tune.lanes_per_row ? 64u : std::max<uint32_t>(G_, 8);
+    const uint32_t G = widen_lanes(c_, G0, R, use_chain ? 32 : 64);
     const TailIO io{rows, R, cnt, res, family_counters(c_, FSIG_K_JOIN_TAIL),
-                    use_chain ? 0u : tail_tile_words(G, L2, c_->tune.lds_tile)};
+                    use_chain ? 0u : tail_tile_words(G, L2, c_->tune.lds_tile),
+                    tail_kids_shared(L1, S1, L2, S2) ? 1u : 0u};
     KTimer t(c_, FSIG_K_JOIN_TAIL);
     int rc = use_chain ? launch_join_tail_chain(c_, G, L1, S1, L2, S2, chain, io)
                        : launch_join_tail(c_, G, L1, S1, L2, S2, io);

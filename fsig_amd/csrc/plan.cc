@@ -192,7 +192,9 @@ void plan_order_gsi(QueryPlan& P, const uint32_t* class_size) {
 // orbit, then fix v) yields conditions that exactly one embedding of every
 // orbit satisfies, and |Aut| is the product of the orbit sizes taken.
 // Automorphic vertices share a refinement class, hence a candidate array,
-// so a condition compares two row words of the same class.
+// so a condition compares two row words of the same class.  A step picks one
+// member of each orbit as the least by some total order; the steps may use
+// different orders, since each speaks of its own vertex and orbit only.
 
 namespace {
 
@@ -229,7 +231,7 @@ struct AutSearch {
 bool plan_symmetry(QueryPlan& P) {
   const uint32_t k = P.k;
   P.aut = 1;
-  for (uint32_t u = 0; u < MAXQ; u++) P.sym_lt[u] = 0;
+  for (uint32_t u = 0; u < MAXQ; u++) P.sym_lt[u] = P.sym_adj[u] = 0;
   AutSearch S(P);
   uint32_t fixed = 0;
   uint32_t lt[MAXQ] = {0};
@@ -265,6 +267,9 @@ bool plan_symmetry(QueryPlan& P) {
     fixed |= 1u << best;
   }
   P.aut = aut;
-  for (uint32_t u = 0; u < k; u++) P.sym_lt[u] = lt[u];
+  for (uint32_t u = 0; u < k; u++) {
+    P.sym_lt[u] = lt[u];
+    if ((lt[u] & ~P.adjm[u]) == 0) P.sym_adj[u] = lt[u];
+  }
   return true;
 }
