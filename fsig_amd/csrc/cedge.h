@@ -86,8 +86,11 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_seg_rows(const PT* __restrict__ 
     if (hub) cnt[f] = 0;
     mine += deg;
   }
-  mine = wave_sum_u64(mine);
-  if ((threadIdx.x & 63u) == 0 && mine) atomicAdd(entries, mine);
+  // one addition per block, and few blocks: additions to one word take 12 ns
+  // each (80 us of a 2^20-row launch when every wavefront made one)
+  __shared__ uint64_t lds[4];
+  mine = block_sum(mine, lds);
+  if (threadIdx.x == 0 && mine) atomicAdd(entries, mine);
 }
 
 // Row, pair and adjacency range of every segment (rows < 2^32), so that a
@@ -332,7 +335,7 @@ int seg_prepare(fsig_ctx* c, const PT* dP, uint32_t np, uint64_t rows, const uin
   unsigned long long* entries = (unsigned long long*)(sr.segbase + rows + 1);
   k_seg_zero<<<1, 64, 0, c->stream>>>(entries);
   const uint64_t blocks = std::min<uint64_t>((rows + FSIG_BLOCK - 1) / FSIG_BLOCK, (uint64_t)c->num_cus * 16);
-  k_seg_rows<PT><<<(uint32_t)blocks, FSIG_BLOCK, 0, c->stream>>>(dP, np, rows, off, nseg, cnt, entries);
+  k_seg_rows<PT><<<(uint32_t)std::min<uint64_t>(blocks, (uint64_t)c->num_cus * 4), FSIG_BLOCK, 0, c->stream>>>(dP, np, rows, off, nseg, cnt, entries);
   FSIG_HIP(c, hipGetLastError());
   int rc;
   if ((rc = scan_u32_to_u64(c, nseg, sr.segbase, rows))) return rc;

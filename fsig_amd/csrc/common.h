@@ -154,12 +154,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_digest(DigestMap M, const uint32
     s0 += x;
     s1 += mix64(x ^ kDigestSalt);
   }
-  s0 = wave_sum_u64(s0);
-  s1 = wave_sum_u64(s1);
-  if ((threadIdx.x & 63u) == 0) {
-    atomicAdd(&acc[0], s0);
-    atomicAdd(&acc[1], s1);
-  }
+  block_add<2>({s0, s1}, {acc, acc + 1});
 }
 
 uint32_t grid_for(const fsig_ctx* c, uint64_t items, uint32_t per_block) {

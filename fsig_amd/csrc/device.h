@@ -6,6 +6,8 @@
 
 #include <cstdint>
 
+#include "internal.h"
+
 #define FSIG_BLOCK 256
 
 // Workgroups are dispatched round-robin over the 8 XCDs of an MI355X, each
@@ -22,6 +24,32 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
+}
+
+// Sums into striped counters (kStripes).  Additions of 64-bit words to one
+// address take 12..13 ns each, one after another, however many compute units
+// send them: with one address and an addition per wavefront and counter, the
+// 16,384 wavefronts of a full launch spent 410 us on two statistics.
+//
+// dst[i], in the block's copy, += the sum of v[i] over the block (dst[i] may
+// be null).  Every thread of the block must call it.
+template <int N>
+__device__ __forceinline__ void block_add(const unsigned long long (&v)[N], unsigned long long* const (&dst)[N]) {
+  __shared__ unsigned long long part[FSIG_BLOCK / 64][N];
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    const unsigned long long s = wave_sum_u64(v[i]);
+    if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6][i] = s;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; i++)
+    if (threadIdx.x == (uint32_t)i && dst[i]) {
+      unsigned long long s = 0;
+#pragma unroll
+      for (int w = 0; w < FSIG_BLOCK / 64; w++) s += part[w][i];
+      if (s) atomicAdd(dst[i] + (blockIdx.x & (kStripes - 1)) * kStripeWords, s);
+    }
 }
 
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }

@@ -898,10 +898,8 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_dfs(const BQuery* __restrict__ Q
       }
     }
   }
-  if (stats && gl == 0) {
-    atomicAdd(&stats[0], (unsigned long long)bytes);
-    atomicAdd(&stats[1], (unsigned long long)nodes);
-  }
+  block_add<2>({stats && gl == 0 ? (unsigned long long)bytes : 0ull, stats && gl == 0 ? (unsigned long long)nodes : 0ull},
+               {stats, stats ? stats + 1 : nullptr});
 }
 
 // ---------------------------------------------------------------------------
@@ -1074,13 +1072,24 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_join_multi(const MLevel* __restr
       }
     }
   }
-  if (!WRITE && gl == 0 && cur_q != 0xffffffffu && acc) atomicAdd(&qcounts[cur_q], acc);
-  my_bytes = wave_sum_u64(my_bytes);
-  my_units = wave_sum_u64(my_units);
-  if (stats && lane == 0) {
-    atomicAdd(&stats[0], my_bytes);
-    atomicAdd(&stats[1], my_units);
+  if (!WRITE) {
+    // what the groups still hold: neighbouring groups end with the same
+    // query, whose counts go out as one addition
+    __shared__ unsigned long long last_acc[GPB];
+    __shared__ uint32_t last_q[GPB];
+    if (gl == 0) {
+      last_acc[gw] = acc;
+      last_q[gw] = acc ? cur_q : 0xffffffffu;
+    }
+    __syncthreads();
+    const uint32_t i = threadIdx.x;
+    if (i < (uint32_t)GPB && last_q[i] != 0xffffffffu && (i == 0 || last_q[i - 1] != last_q[i])) {
+      unsigned long long s = 0;
+      for (uint32_t j = i; j < (uint32_t)GPB && last_q[j] == last_q[i]; j++) s += last_acc[j];
+      atomicAdd(&qcounts[last_q[i]], s);
+    }
   }
+  block_add<2>({my_bytes, my_units}, {stats, stats ? stats + 1 : nullptr});
 }
 
 __global__ void k_iota_multi(const uint64_t* __restrict__ qbase, uint32_t nlive, uint32_t* __restrict__ rows,
@@ -2032,7 +2041,12 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
       k_iota_multi<<<bgrid(c, R, FSIG_BLOCK), FSIG_BLOCK, 0, c->stream>>>(dqb, nl, rows, R);
       std::vector<MLevel> ml(nl);
       uint64_t prev_bytes = 0;  // debug timing: device byte counter before the level
-      if (clk.on && stats_ls) (void)read_u64(c, stats_ls, &prev_bytes, 1);
+      auto level_bytes = [&]() -> uint64_t {
+        uint64_t w[2 * FSIG_K_BATCH + 1] = {0};
+        (void)read_striped(c, c->d_counters + kStripes * kStripeWords, w, 2 * FSIG_K_BATCH + 1);
+        return w[2 * FSIG_K_BATCH];
+      };
+      if (clk.on) prev_bytes = level_bytes();
       // one launch per lane-count group over its row range of the level
       auto launch = [&](bool write, uint32_t p, uint32_t* cnt, uint64_t* off, uint32_t* out) -> int {
         for (size_t gi = 0; gi + 1 < gstart.size(); gi++) {
@@ -2064,7 +2078,7 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
       for (uint32_t p = 1; p < maxk && R > 0; p++) {
         if (clk.on) {
           clk.mark("lockstep level start");
-          if (stats_ls) (void)read_u64(c, stats_ls, &prev_bytes, 1);
+          prev_bytes = level_bytes();
         }
         bool any_more = false;
         make_groups(p);
@@ -2087,11 +2101,8 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
           return rc2;
         }
         if (clk.on) {
-          uint64_t st2[2] = {0, 0};
-          if (stats_ls && read_u64(c, stats_ls, st2, 2) == FSIG_OK) {
-            fprintf(stderr, "[fsig batch]   level %u: %llu rows -> %llu, count-pass bytes/row %.1f\n", p,
-                    (unsigned long long)R, (unsigned long long)T, R ? (double)(st2[0] - prev_bytes) / R : 0.0);
-          }
+          fprintf(stderr, "[fsig batch]   level %u: %llu rows -> %llu, count-pass bytes/row %.1f\n", p,
+                  (unsigned long long)R, (unsigned long long)T, R ? (double)(level_bytes() - prev_bytes) / R : 0.0);
           clk.mark("  count + scan");
         }
         if (T == 0) break;

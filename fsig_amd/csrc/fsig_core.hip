@@ -108,14 +108,31 @@ int resolve_timings(fsig_ctx* c) {
     c->kstat[c->timed[i].fam].ms += ms;
   }
   c->timed_used = 0;
-  uint64_t fam[4 * FSIG_K_NUM];
-  int rc = read_u64(c, c->d_counters + 16, fam, 4 * FSIG_K_NUM);
+  constexpr size_t kWords = kStripes * kStripeWords;
+  uint64_t fam[kWords];
+  int rc = read_u64(c, c->d_counters + kWords, fam, kWords);
   if (rc) return rc;
-  for (int f = 0; f < FSIG_K_NUM; f++) {
-    c->kstat[f].alg_bytes += fam[4 * f];
-    c->kstat[f].units += fam[4 * f + 1];
-  }
-  FSIG_HIP(c, hipMemsetAsync(c->d_counters + 16, 0, 8 * 4 * FSIG_K_NUM, c->stream));
+  for (uint32_t s = 0; s < kStripes; s++)
+    for (int f = 0; f < FSIG_K_NUM; f++) {
+      c->kstat[f].alg_bytes += fam[s * kStripeWords + 2 * f];
+      c->kstat[f].units += fam[s * kStripeWords + 2 * f + 1];
+    }
+  FSIG_HIP(c, hipMemsetAsync(c->d_counters + kWords, 0, 8 * kWords, c->stream));
+  return FSIG_OK;
+}
+
+int clear_results(fsig_ctx* c) {
+  FSIG_HIP(c, hipMemsetAsync(c->d_counters, 0, 8 * kStripes * kStripeWords, c->stream));
+  return FSIG_OK;
+}
+
+int read_striped(fsig_ctx* c, const unsigned long long* dev, uint64_t* host, uint32_t n) {
+  uint64_t all[kStripes * kStripeWords];
+  const int rc = read_u64(c, dev, all, kStripes * kStripeWords);
+  if (rc) return rc;
+  for (uint32_t i = 0; i < n; i++) host[i] = 0;
+  for (uint32_t s = 0; s < kStripes; s++)
+    for (uint32_t i = 0; i < n; i++) host[i] += all[s * kStripeWords + i];
   return FSIG_OK;
 }
 
@@ -174,7 +191,7 @@ int fsig_ctx_create(int device, uint64_t budget, fsig_ctx** out) {
   if (budget > freeb) { delete c; return FSIG_ENOMEM; }
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&c->ev_a) != hipSuccess || hipEventCreate(&c->ev_b) != hipSuccess ||
-      hipMalloc((void**)&c->d_counters, 64 * sizeof(unsigned long long)) != hipSuccess ||
+      hipMalloc((void**)&c->d_counters, kCounterWords * sizeof(unsigned long long)) != hipSuccess ||
       hipHostMalloc((void**)&c->h_pinned, kPinnedWords * 8, hipHostMallocDefault) != hipSuccess) {
     fsig_ctx_destroy(c);
     return FSIG_EHIP;
@@ -184,7 +201,7 @@ int fsig_ctx_create(int device, uint64_t budget, fsig_ctx** out) {
     return FSIG_ENOMEM;
   }
   c->arena.cap = budget;
-  if (hipMemset(c->d_counters, 0, 64 * sizeof(unsigned long long)) != hipSuccess) {
+  if (hipMemset(c->d_counters, 0, kCounterWords * sizeof(unsigned long long)) != hipSuccess) {
     fsig_ctx_destroy(c);
     return FSIG_EHIP;
   }
@@ -395,9 +412,9 @@ static int match_impl(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
   c->arena.peak = mk;
   unsigned long long* acc = nullptr;
   if (digest_out) {
-    acc = (unsigned long long*)c->arena.alloc(2 * sizeof(unsigned long long));
+    acc = (unsigned long long*)c->arena.alloc(8ull * kStripes * kStripeWords);
     if (!acc) return set_err(c, FSIG_ENOMEM, "digest: arena exhausted");
-    k_fill_words<<<1, 64, 0, c->stream>>>((uint32_t*)acc, 4);
+    k_fill_words<<<1, FSIG_BLOCK, 0, c->stream>>>((uint32_t*)acc, 2 * kStripes * kStripeWords);
     FSIG_HIP(c, hipGetLastError());
   }
   // A count counts one embedding per orbit of the query's automorphisms
@@ -425,7 +442,7 @@ static int match_impl(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
     *count_out = orbits > UINT64_MAX / P.aut ? UINT64_MAX : orbits * P.aut;
     if (max_emb) *count_out = std::min(*count_out, max_emb);
   }
-  if (rc == FSIG_OK && acc) rc = read_u64(c, acc, digest_out, 2);
+  if (rc == FSIG_OK && acc) rc = read_striped(c, acc, digest_out, 2);
   c->last_peak = c->arena.peak - mk;
   c->arena.release(mk);
   hipError_t e = hipStreamSynchronize(c->stream);
@@ -458,8 +475,10 @@ int fsig_match_digest(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
 // holds its own copy until the process ends.  In host code `scratch` names a
 // host-side stand-in, never the device memory: its device address is taken
 // once per device with hipGetSymbolAddress and only that address is used.
-constexpr size_t kScratchCounters = 64 * sizeof(unsigned long long);
-static __device__ __align__(256) char scratch[FSIG_NOALLOC_SCRATCH_BYTES];
+// Of the promised bytes, 512 are the engine's own; its counters follow the
+// array's end.
+constexpr size_t kScratchOwn = 512;
+static __device__ __align__(256) char scratch[FSIG_NOALLOC_SCRATCH_BYTES + kCounterWords * sizeof(unsigned long long)];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -493,7 +512,7 @@ int fsig_match_noalloc(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32
   // the candidate mask (4 bytes a vertex) and the candidate arrays (at most
   // 4 bytes a vertex of the query's labels, twice) must fit with room left
   const uint64_t need = 12ull * g->n + (1u << 20);
-  if (need > FSIG_NOALLOC_SCRATCH_BYTES - kScratchCounters)
+  if (need > FSIG_NOALLOC_SCRATCH_BYTES - kScratchOwn)
     return set_err(c, FSIG_EINVAL,
                    "noalloc: a graph of " + std::to_string(g->n) + " vertices needs at least " +
                        std::to_string(need) + " bytes of scratch, more than the static " +
@@ -506,16 +525,16 @@ int fsig_match_noalloc(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32
   Arena saved_arena = c->arena;
   unsigned long long* saved_counters = c->d_counters;
   const bool saved_prof = c->profiling;
-  c->d_counters = (unsigned long long*)base;
+  c->d_counters = (unsigned long long*)(base + FSIG_NOALLOC_SCRATCH_BYTES);
   c->arena = Arena();
-  c->arena.base = base + kScratchCounters;
-  c->arena.cap = FSIG_NOALLOC_SCRATCH_BYTES - kScratchCounters;
+  c->arena.base = base + kScratchOwn;
+  c->arena.cap = FSIG_NOALLOC_SCRATCH_BYTES - kScratchOwn;
   c->profiling = false;
   rc = FSIG_OK;
   // the counters must start at zero: earlier calls leave theirs behind
   if (hipSetDevice(c->device) != hipSuccess) rc = set_err(c, FSIG_EHIP, "noalloc: hipSetDevice failed");
   if (rc == FSIG_OK) {
-    k_fill_words<<<1, 64, 0, c->stream>>>((uint32_t*)base, (uint32_t)(kScratchCounters / 4));
+    k_fill_words<<<1, FSIG_BLOCK, 0, c->stream>>>((uint32_t*)c->d_counters, (uint32_t)(2 * kCounterWords));
     if (hipGetLastError() != hipSuccess) rc = set_err(c, FSIG_EHIP, "noalloc: clearing the scratch counters failed");
   }
   if (rc == FSIG_OK)

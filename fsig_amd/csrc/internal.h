@@ -14,6 +14,11 @@
 #define MAXQ 32
 constexpr size_t kPinnedWords = 65536;
 #define FSIG_INVALID 0xffffffffu
+// Device counters are kept in kStripes copies of kStripeWords words (one
+// cache line) each: a block adds to the copy of its number (block_add) and
+// the host sums them.
+constexpr uint32_t kStripes = 32;
+constexpr uint32_t kStripeWords = 16;
 
 // ---------------------------------------------------------------------------
 // Device-memory arena: one hipMalloc per context, bump allocation with
@@ -73,9 +78,10 @@ struct fsig_ctx {
   bool keep_cand = false;
   std::vector<std::vector<uint32_t>> cand_sets[2];
   uint64_t last_peak = 0;
-  // device counters (64 words): [0..7] per-launch results, [16 + 4f ..] per
-  // kernel family f accumulated device-side statistics ([0] algorithmic
-  // bytes, [1] units).  Host staging is pinned.
+  // device counters, kCounterWords: kStripes copies of kStripeWords words for
+  // per-launch results, then as many for the statistics accumulated per
+  // kernel family f (word 2f algorithmic bytes, 2f+1 units); see block_add.
+  // Host staging is pinned.
   unsigned long long* d_counters = nullptr;
   unsigned long long* h_pinned = nullptr;  // kPinnedWords words of pinned staging
   int num_cus = 256;
@@ -204,7 +210,15 @@ struct KTimer {
 // Adds the recorded event intervals and the device-side family counters into
 // the context statistics; the stream must be idle.
 int resolve_timings(fsig_ctx* c);
-inline unsigned long long* family_counters(fsig_ctx* c, int fam) { return c->d_counters + 16 + 4 * fam; }
+static_assert(2 * FSIG_K_NUM <= (int)kStripeWords, "the families' counters fit one copy");
+constexpr size_t kCounterWords = 2 * kStripes * kStripeWords;
+inline unsigned long long* family_counters(fsig_ctx* c, int fam) {
+  return c->d_counters + kStripes * kStripeWords + 2 * fam;
+}
+// Zeroes the per-launch results (on the stream) / reads the sums of the
+// first n words of striped counters.
+int clear_results(fsig_ctx* c);
+int read_striped(fsig_ctx* c, const unsigned long long* dev, uint64_t* host, uint32_t n);
 // Refinement passes: the tuned cap, else 2 (one query or a batch).  After
 // the neighbour-label filter the second pass still pays for itself on large
 // graphs (smaller candidate edges and joins); later ones remove a few
@@ -219,7 +233,7 @@ int scan_u32_to_u64(fsig_ctx* c, const uint32_t* in, uint64_t* out, uint64_t n);
 int read_u64(fsig_ctx* c, const void* dev, uint64_t* host, size_t count);
 
 // The per-query matcher pipelines.
-// digest_acc (two zeroed device words, may be null): enumerate every
+// digest_acc (two zeroed striped counters, may be null): enumerate every
 // embedding and fold it into the order-independent set digest there instead
 // of copying rows to emb_out.
 // by_degree: symmetry conditions between neighbours (P.sym_adj) order them by

@@ -305,16 +305,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_join(JoinLevel L, Src S, JoinIO 
       my_bytes += b;
     }
   }
-  my_children = wave_sum_u64(my_children);
-  my_bytes = wave_sum_u64(my_bytes);
-  my_rows = wave_sum_u64(my_rows);
-  if (lane == 0) {
-    if (!WRITE && io.total) atomicAdd(io.total, my_children);
-    if (io.stats) {
-      atomicAdd(&io.stats[0], my_bytes);
-      atomicAdd(&io.stats[1], my_rows);
-    }
-  }
+  block_add<3>({my_children, my_bytes, my_rows}, {WRITE ? nullptr : io.total, io.stats, io.stats ? io.stats + 1 : nullptr});
 }
 
 // ---------------------------------------------------------------------------
@@ -815,18 +806,7 @@ k_join_tail(JoinLevel L1, CandEdgeSrc S1, JoinLevel L2, CandEdgeSrc S2, TailIO i
       my_rows += 1;
     }
   }
-  my_leaves = wave_sum_u64(my_leaves);
-  my_kids = wave_sum_u64(my_kids);
-  my_bytes = wave_sum_u64(my_bytes);
-  my_rows = wave_sum_u64(my_rows);
-  if (lane == 0) {
-    atomicAdd(&io.res[0], my_leaves);
-    atomicAdd(&io.res[1], my_kids);
-    if (io.stats) {
-      atomicAdd(&io.stats[0], my_bytes);
-      atomicAdd(&io.stats[1], my_rows);
-    }
-  }
+  block_add<4>({my_leaves, my_kids, my_bytes, my_rows}, {io.res, io.res + 1, io.stats, io.stats ? io.stats + 1 : nullptr});
 }
 
 // Whether the fused tail applies to leaf level L2: it needs a backward list,
@@ -1040,18 +1020,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_join_tail_chain(JoinLevel L1, Ca
       my_rows += 1;
     }
   }
-  my_leaves = wave_sum_u64(my_leaves);
-  my_kids = wave_sum_u64(my_kids);
-  my_bytes = wave_sum_u64(my_bytes);
-  my_rows = wave_sum_u64(my_rows);
-  if (lane == 0) {
-    atomicAdd(&io.res[0], my_leaves);
-    atomicAdd(&io.res[1], my_kids);
-    if (io.stats) {
-      atomicAdd(&io.stats[0], my_bytes);
-      atomicAdd(&io.stats[1], my_rows);
-    }
-  }
+  block_add<4>({my_leaves, my_kids, my_bytes, my_rows}, {io.res, io.res + 1, io.stats, io.stats ? io.stats + 1 : nullptr});
 }
 
 // Whether the chain tail applies to levels p (L1) and p+1 (L2).
@@ -1219,13 +1188,13 @@ class JoinDriver {
       fused = mode_ == FSIG_MODE_COUNT && p + 2 == k_ && c_->tune.fused_tail == 0 && tail_applies(pv_.level(p + 1)) &&
               L.nb <= kTailMax && L.ncf <= kTailMax;
     if (last && mode_ == FSIG_MODE_COUNT) {
-      FSIG_HIP(c_, hipMemsetAsync(res, 0, sizeof(unsigned long long), c_->stream));
+      if ((rc = clear_results(c_))) return rc;
       JoinIO io{rows, 0, R, nullptr, nullptr, nullptr, 0, 0, res, family_counters(c_, FSIG_K_JOIN_COUNT)};
       KTimer t(c_, FSIG_K_JOIN_COUNT);
       if ((rc = launch_join<false>(c_, widen_lanes(c_, G_, R, 64), L, S, io))) return rc;
       t.done(0, 0);
       uint64_t h;
-      if ((rc = read_u64(c_, res, &h, 1))) return rc;
+      if ((rc = read_striped(c_, res, &h, 1))) return rc;
       total_ += std::min(h, remaining());
       return FSIG_OK;
     }
@@ -1316,7 +1285,8 @@ class JoinDriver {
   int count_tail(const uint32_t* rows, uint64_t R, uint32_t* cnt, const JoinLevel& L1, const CandEdgeSrc& S1,
                  const JoinLevel& L2, const CandEdgeSrc& S2) {
     unsigned long long* res = c_->d_counters;
-    FSIG_HIP(c_, hipMemsetAsync(res, 0, 2 * sizeof(unsigned long long), c_->stream));
+    int rc = clear_results(c_);
+    if (rc) return rc;
     ChainTail chain;
     const bool use_chain = chain_tail_applies(L1, L2) && pv_.chain_tail(L1.p, chain);
     // lanes per parent row: at least 8 where the shared intersection goes
@@ -1332,12 +1302,12 @@ class JoinDriver {
                     use_chain ? 0u : tail_tile_words(G, L2, c_->tune.lds_tile),
                     tail_kids_shared(L1, S1, L2, S2) ? 1u : 0u};
     KTimer t(c_, FSIG_K_JOIN_TAIL);
-    int rc = use_chain ? launch_join_tail_chain(c_, G, L1, S1, L2, S2, chain, io)
+    rc = use_chain ? launch_join_tail_chain(c_, G, L1, S1, L2, S2, chain, io)
                        : launch_join_tail(c_, G, L1, S1, L2, S2, io);
     if (rc) return rc;
     t.done(0, 0);
     uint64_t h[2];
-    if ((rc = read_u64(c_, res, h, 2))) return rc;
+    if ((rc = read_striped(c_, res, h, 2))) return rc;
     rows_ += h[1];
     const uint64_t limit = c_->work_limit;
     if (limit && rows_ > limit) return set_err(c_, FSIG_ELIMIT, "join: work limit exceeded");
