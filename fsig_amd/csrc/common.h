@@ -132,16 +132,10 @@ __global__ void k_emit(EmitMap M, const uint32_t* __restrict__ rows, uint64_t n,
 }
 
 // Digest of level-k rows: one row per thread, words taken in query-vertex
-// order (join position M.pos[i] holds query vertex i); per-wave sums are
-// added to acc[0..1].
-struct DigestMap {
-  uint32_t k;
-  uint32_t pos[MAXQ];             // join position of query vertex i
-  const uint32_t* cand[MAXQ];     // candidate array of join position c (null: word is a vertex id)
-};
-
-__global__ void __launch_bounds__(FSIG_BLOCK) k_digest(DigestMap M, const uint32_t* __restrict__ rows, uint64_t n,
-                                                       unsigned long long* __restrict__ acc) {
+// order; per-wave sums are added to M.acc[0..1].  A match's last level is
+// digested as it is found (k_join); this takes tables that are there already
+// (a query of one vertex, a bounded match).
+__global__ void __launch_bounds__(FSIG_BLOCK) k_digest(DigestMap M, const uint32_t* __restrict__ rows, uint64_t n) {
   unsigned long long s0 = 0, s1 = 0;
   for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t* row = rows + r * M.k;
@@ -154,7 +148,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_digest(DigestMap M, const uint32
     s0 += x;
     s1 += mix64(x ^ kDigestSalt);
   }
-  block_add<2>({s0, s1}, {acc, acc + 1});
+  block_add<2>({s0, s1}, {M.acc, M.acc + 1});
 }
 
 uint32_t grid_for(const fsig_ctx* c, uint64_t items, uint32_t per_block) {
@@ -191,10 +185,10 @@ struct HostSink : LeafSink {
 struct DigestSink : LeafSink {
   fsig_ctx* c;
   DigestMap map;
-  unsigned long long* acc;
+  const DigestMap* digest() const override { return &map; }
   int take(const uint32_t* rows, uint64_t n) override {
     if (n == 0) return FSIG_OK;
-    k_digest<<<grid_for(c, n, FSIG_BLOCK), FSIG_BLOCK, 0, c->stream>>>(map, rows, n, acc);
+    k_digest<<<grid_for(c, n, FSIG_BLOCK), FSIG_BLOCK, 0, c->stream>>>(map, rows, n);
     FSIG_HIP(c, hipGetLastError());
     return FSIG_OK;
   }
@@ -215,11 +209,12 @@ struct LeafSinks {
     digest.c = c;
     std::memset(&digest.map, 0, sizeof(digest.map));
     digest.map.k = k;
-    digest.acc = digest_acc;
+    digest.map.acc = digest_acc;
     for (uint32_t p = 0; p < k; p++) {
       host.map.qv[p] = order[p];
       host.map.cand[p] = cand_of_pos ? cand_of_pos[p] : nullptr;
       digest.map.pos[order[p]] = p;
+      digest.map.qv[p] = order[p];
       digest.map.cand[p] = cand_of_pos ? cand_of_pos[p] : nullptr;
     }
     host.host = emb_out;

@@ -176,19 +176,52 @@ __device__ __forceinline__ uint32_t group_col(const uint32_t (&rv)[(MAXQ + G - 1
   return __shfl(v, (int)(c % G), G);
 }
 
-// WRITE == false: count pass (children per row into io.cnt, total into
-// counters[0]).  WRITE == true: children of rows [row_lo, row_hi) whose global
-// index falls in [out_lo, out_hi) are written as p+1 word rows.
-template <int G, bool WRITE, class Src>
-__global__ void __launch_bounds__(FSIG_BLOCK) k_join(JoinLevel L, Src S, JoinIO io) {
+// How a row of level k is folded into the set digest: words in query-vertex
+// order, sums added to the striped counters acc[0..1].
+struct DigestMap {
+  uint32_t k;
+  uint32_t pos[MAXQ];          // join position of query vertex i
+  uint32_t qv[MAXQ];           // query vertex of join position c
+  const uint32_t* cand[MAXQ];  // candidate array of join position c (null: word is a vertex id)
+  unsigned long long* acc;
+};
+
+// Count: children per row into io.cnt (may be null), their number into
+// io.total.  Write: children of rows [row_lo, row_hi) whose global index
+// falls in [out_lo, out_hi) are written as p+1 word rows.  Digest (the last
+// level): every child completes an embedding, which is folded into the set
+// digest and written nowhere; their number into io.total.
+enum JoinMode : int { kJoinCount = 0, kJoinWrite = 1, kJoinDigest = 2 };
+struct NoDigest {};
+template <int MODE>
+using DigestArg = typename std::conditional<MODE == kJoinDigest, DigestMap, NoDigest>::type;
+
+// Orders the LDS accesses of one wavefront (no workgroup barrier needed).
+__device__ __forceinline__ void lds_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The digest is bound by its hash chain (two 64-bit products a word), which
+// runs over a row's words in query-vertex order: the words before the new
+// vertex are the same for every child and are hashed once per row.
+// Written and read back by a kernel of its own, each 32-byte row cost more
+// than its hash: the 8-vertex dense query's set on the 200,001-vertex dblp-law
+// graph took 14.3 ms and takes 1.7 ms.
+template <int G, int MODE, class Src>
+__global__ void __launch_bounds__(FSIG_BLOCK) k_join(JoinLevel L, Src S, JoinIO io, DigestArg<MODE> D) {
+  constexpr bool WRITE = MODE == kJoinWrite, DIGEST = MODE == kJoinDigest;
   constexpr int GPB = FSIG_BLOCK / G;  // groups per block
   constexpr int NR = (MAXQ + G - 1) / G;
   __shared__ uint32_t sh_s[GPB][MAXQ];
   __shared__ uint32_t sh_n[GPB][MAXQ];
   __shared__ uint32_t sh_cf[GPB][MAXQ];
+  __shared__ uint32_t sh_id[DIGEST ? GPB : 1][MAXQ];  // the row's data vertices, by query vertex
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t gl = lane & (G - 1);
   const uint32_t gw = threadIdx.x / G;
+  unsigned long long dig0 = 0, dig1 = 0;
   const uint64_t gmask = (G == 64) ? ~0ull : (((1ull << G) - 1) << (lane - gl));
   const uint64_t below = (1ull << lane) - 1;
   const uint64_t ngroups = (uint64_t)gridDim.x * GPB;
@@ -219,6 +252,18 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_join(JoinLevel L, Src S, JoinIO 
       if (!((L.cfsame >> j) & 1u)) x = L.cfcand[j][x];
       sh_cf[gw][j] = x;
     }
+    uint64_t prefix = 0;
+    if constexpr (DIGEST) {
+      lds_wave_sync();  // the previous row's reads
+#pragma unroll
+      for (int j = 0; j < NR; j++) {
+        const uint32_t col = j * G + gl;
+        if (col < L.p) sh_id[gw][D.qv[col]] = D.cand[col] ? D.cand[col][rv[j]] : rv[j];
+      }
+      lds_wave_sync();
+      prefix = row_hash_start(D.k);
+      for (uint32_t i = 0; i < D.qv[L.p]; i++) prefix = row_hash_step(prefix, i, sh_id[gw][i]);
+    }
     uint64_t base = 0;
     uint64_t child0 = 0;
     if (WRITE) {
@@ -236,7 +281,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_join(JoinLevel L, Src S, JoinIO 
     // Count pass with one backward list of candidates only: the children are
     // the list minus the earlier vertices of the same label that occur in
     // it, found by binary search (one lane per conflict).
-    const bool direct = !WRITE && Src::kAllMembers && L.nb == 1;
+    const bool direct = MODE == kJoinCount && Src::kAllMembers && L.nb == 1;
     if (direct) {
       uint32_t hit = 0;
       for (uint32_t j0 = 0; j0 < L.ncf; j0 += G) {
@@ -280,6 +325,15 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_join(JoinLevel L, Src S, JoinIO 
         }
         if (put) dst[L.p] = x;
       }
+      if constexpr (DIGEST) {
+        if (ok) {
+          const uint32_t q = D.qv[L.p];
+          uint64_t h = row_hash_step(prefix, q, D.cand[L.p] ? D.cand[L.p][x] : x);
+          for (uint32_t i = q + 1; i < D.k; i++) h = row_hash_step(h, i, sh_id[gw][i]);
+          dig0 += h;
+          dig1 += mix64(h ^ kDigestSalt);
+        }
+      }
       base += __popcll(bal);
     }
     if (!WRITE && io.cnt && gl == 0) io.cnt[r] = (uint32_t)base;
@@ -305,6 +359,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_join(JoinLevel L, Src S, JoinIO 
       my_bytes += b;
     }
   }
+  if constexpr (DIGEST) block_add<2>({dig0, dig1}, {D.acc, D.acc + 1});
   block_add<3>({my_children, my_bytes, my_rows}, {WRITE ? nullptr : io.total, io.stats, io.stats ? io.stats + 1 : nullptr});
 }
 
@@ -342,12 +397,6 @@ struct TailLds {
   uint32_t* tile;  // tw words
   uint32_t tw;
 };
-
-__device__ __forceinline__ void lds_wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Lists of the leaf level: only shared ones (of parent columns), only the
 // child's own, or both.
@@ -1069,8 +1118,9 @@ static __global__ void k_window_rows(const uint64_t* __restrict__ off, uint64_t 
 }
 
 // Host launcher for the join kernel, dispatching on G.
-template <bool WRITE, class Src>
-int launch_join(fsig_ctx* c, uint32_t G, const JoinLevel& L, const Src& S, const JoinIO& io) {
+template <int MODE, class Src>
+int launch_join(fsig_ctx* c, uint32_t G, const JoinLevel& L, const Src& S, const JoinIO& io,
+                const DigestArg<MODE>& D = DigestArg<MODE>()) {
   const uint64_t nrows = io.row_hi - io.row_lo;
   if (nrows == 0) return FSIG_OK;
   const uint64_t gpb = FSIG_BLOCK / G;
@@ -1080,11 +1130,11 @@ int launch_join(fsig_ctx* c, uint32_t G, const JoinLevel& L, const Src& S, const
   if (blocks >= 64) blocks &= ~7ull;  // whole multiples of 8 XCDs
   const uint32_t grid = (uint32_t)std::max<uint64_t>(blocks, 1);
   switch (G) {
-    case 4: k_join<4, WRITE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io); break;
-    case 8: k_join<8, WRITE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io); break;
-    case 16: k_join<16, WRITE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io); break;
-    case 32: k_join<32, WRITE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io); break;
-    default: k_join<64, WRITE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io); break;
+    case 4: k_join<4, MODE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io, D); break;
+    case 8: k_join<8, MODE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io, D); break;
+    case 16: k_join<16, MODE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io, D); break;
+    case 32: k_join<32, MODE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io, D); break;
+    default: k_join<64, MODE, Src><<<grid, FSIG_BLOCK, 0, c->stream>>>(L, S, io, D); break;
   }
   FSIG_HIP(c, hipGetLastError());
   return FSIG_OK;
@@ -1094,6 +1144,8 @@ int launch_join(fsig_ctx* c, uint32_t G, const JoinLevel& L, const Src& S, const
 struct LeafSink {
   virtual ~LeafSink() = default;
   virtual int take(const uint32_t* rows, uint64_t n) = 0;
+  // the digest every embedding goes to, when that is all the sink wants
+  virtual const DigestMap* digest() const { return nullptr; }
 };
 
 // Lanes per row of a launch over R parent rows: G, doubled while the launch
@@ -1191,11 +1243,24 @@ class JoinDriver {
       if ((rc = clear_results(c_))) return rc;
       JoinIO io{rows, 0, R, nullptr, nullptr, nullptr, 0, 0, res, family_counters(c_, FSIG_K_JOIN_COUNT)};
       KTimer t(c_, FSIG_K_JOIN_COUNT);
-      if ((rc = launch_join<false>(c_, widen_lanes(c_, G_, R, 64), L, S, io))) return rc;
+      if ((rc = launch_join<kJoinCount>(c_, widen_lanes(c_, G_, R, 64), L, S, io))) return rc;
       t.done(0, 0);
       uint64_t h;
       if ((rc = read_striped(c_, res, &h, 1))) return rc;
       total_ += std::min(h, remaining());
+      return FSIG_OK;
+    }
+    if (const DigestMap* D = last && sink_ && !bounded() ? sink_->digest() : nullptr) {
+      // every child is an embedding and is only digested: no offsets, no
+      // table, no second pass
+      if ((rc = clear_results(c_))) return rc;
+      JoinIO io{rows, 0, R, nullptr, nullptr, nullptr, 0, 0, res, family_counters(c_, FSIG_K_JOIN_COUNT)};
+      KTimer t(c_, FSIG_K_JOIN_COUNT);
+      if ((rc = launch_join<kJoinDigest>(c_, widen_lanes(c_, G_, R, 64), L, S, io, *D))) return rc;
+      t.done(0, 0);
+      uint64_t h;
+      if ((rc = read_striped(c_, res, &h, 1))) return rc;
+      total_ += h;
       return FSIG_OK;
     }
     uint32_t* cnt = (uint32_t*)c_->arena.alloc(4 * R);
@@ -1211,7 +1276,7 @@ class JoinDriver {
     if (!fused) {
       JoinIO io{rows, 0, R, cnt, nullptr, nullptr, 0, 0, nullptr, family_counters(c_, FSIG_K_JOIN_COUNT)};
       KTimer t(c_, FSIG_K_JOIN_COUNT);
-      if ((rc = launch_join<false>(c_, widen_lanes(c_, G_, R, 64), L, S, io))) return rc;
+      if ((rc = launch_join<kJoinCount>(c_, widen_lanes(c_, G_, R, 64), L, S, io))) return rc;
       t.done(0, 0);
     }
     if ((rc = scan_u32_to_u64(c_, cnt, off, R))) return rc;
@@ -1268,7 +1333,7 @@ class JoinDriver {
                 family_counters(c_, FSIG_K_JOIN_WRITE)};
       {
         KTimer t(c_, FSIG_K_JOIN_WRITE);
-        if ((rc = launch_join<true>(c_, widen_lanes(c_, G_, win[1] - win[0], 64), L, S, io))) return rc;
+        if ((rc = launch_join<kJoinWrite>(c_, widen_lanes(c_, G_, win[1] - win[0], 64), L, S, io))) return rc;
         t.done(0, 0);
       }
       if ((rc = expand(p + 1, child, hi - lo))) return rc;
