@@ -1295,6 +1295,15 @@ class JoinDriver {
       fused = mode_ == FSIG_MODE_COUNT && p + 2 == k_ && c_->tune.fused_tail == 0 && tail_applies(pv_.level(p + 1)) &&
               L.nb <= kTailMax && L.ncf <= kTailMax;
     if (last && mode_ == FSIG_MODE_COUNT) {
+      if constexpr (std::is_same<Src, PcsrSrc>::value) {
+        bool counted = false;
+        uint64_t h = 0;
+        if ((rc = pv_.count_leaves(c_, G_, p, L, S, rows, R, counted, h))) return rc;
+        if (counted) {
+          total_ += std::min(h, remaining());
+          return FSIG_OK;
+        }
+      }
       if ((rc = clear_results(c_))) return rc;
       JoinIO io{rows, 0, R, nullptr, nullptr, nullptr, 0, 0, res, family_counters(c_, FSIG_K_JOIN_COUNT)};
       KTimer t(c_, FSIG_K_JOIN_COUNT);
