@@ -321,11 +321,13 @@ struct SegRows {
   uint32_t* seg_pair = nullptr;
   uint2* seg_range = nullptr;  // adjacency entries [x, y) of the segment
   uint64_t nsegs = 0;
-  uint64_t entries = 0;  // adjacency entries of all rows
+  uint64_t entries = 0;  // adjacency entries of all rows (with hubs; on the device at segbase[rows + 1])
 };
 
+// hubs: whether the graph has a vertex of more than kHubDeg neighbours; with
+// none there is no segment to number and nothing to wait for.
 template <class PT>
-int seg_prepare(fsig_ctx* c, const PT* dP, uint32_t np, uint64_t rows, const uint32_t* off, uint32_t* cnt,
+int seg_prepare(fsig_ctx* c, const PT* dP, uint32_t np, uint64_t rows, const uint32_t* off, uint32_t* cnt, bool hubs,
                 SegRows& sr) {
   if (rows == 0) return FSIG_OK;
   if (rows >= 0xffffffffull) return set_err(c, FSIG_EUNSUPPORTED, "cedge: too many candidate rows");
@@ -337,6 +339,7 @@ int seg_prepare(fsig_ctx* c, const PT* dP, uint32_t np, uint64_t rows, const uin
   const uint64_t blocks = std::min<uint64_t>((rows + FSIG_BLOCK - 1) / FSIG_BLOCK, (uint64_t)c->num_cus * 16);
   k_seg_rows<PT><<<(uint32_t)std::min<uint64_t>(blocks, (uint64_t)c->num_cus * 4), FSIG_BLOCK, 0, c->stream>>>(dP, np, rows, off, nseg, cnt, entries);
   FSIG_HIP(c, hipGetLastError());
+  if (!hubs) return FSIG_OK;
   int rc;
   if ((rc = scan_u32_to_u64(c, nseg, sr.segbase, rows))) return rc;
   uint64_t tail[2];

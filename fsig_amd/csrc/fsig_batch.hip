@@ -1676,7 +1676,7 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
     if (!dP || !dS || (!bt.empty() && !dbt) || !cnt || !gscan || !dmax || !pb)
       return set_err(c, FSIG_ENOMEM, "batch: arena exhausted");
     SegRows segs;  // hub rows of every pair, one wavefront per segment
-    if ((rc = seg_prepare(c, dP, np, pflat, g->d_off, cnt, segs))) return rc;
+    if ((rc = seg_prepare(c, dP, np, pflat, g->d_off, cnt, true, segs))) return rc;
     // the chunks' source, pair-row and segment ranges
     const size_t nch = use_bits ? chunk_q.size() : 1;
     std::vector<uint64_t> ch_src(nch + 1), ch_row(nch + 1), ch_seg(nch + 1, 0);
@@ -2305,7 +2305,7 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
   c->last_tune_engine = best.lockstep ? 1 : 2;
   c->last_peak = A.peak - mark;
   FSIG_HIP(c, hipStreamSynchronize(c->stream));
-  return resolve_timings(c);
+  return resolve_events(c);
 }
 
 extern "C" int fsig_match_batch(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint32_t* ks,

@@ -101,13 +101,17 @@ int scan_u32_to_u64(fsig_ctx* c, const uint32_t* in, uint64_t* out, uint64_t n) 
   return FSIG_OK;
 }
 
-int resolve_timings(fsig_ctx* c) {
+int resolve_events(fsig_ctx* c) {
   for (size_t i = 0; i < c->timed_used; i++) {
     float ms = 0;
     FSIG_HIP(c, hipEventElapsedTime(&ms, c->timed[i].a, c->timed[i].b));
     c->kstat[c->timed[i].fam].ms += ms;
   }
   c->timed_used = 0;
+  return FSIG_OK;
+}
+
+int fetch_stats(fsig_ctx* c) {
   constexpr size_t kWords = kStripes * kStripeWords;
   uint64_t fam[kWords];
   int rc = read_u64(c, c->d_counters + kWords, fam, kWords);
@@ -447,7 +451,7 @@ static int match_impl(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
   c->arena.release(mk);
   hipError_t e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) return set_err(c, FSIG_EHIP, std::string("match: ") + hipGetErrorString(e));
-  int rt = resolve_timings(c);
+  int rt = resolve_events(c);
   return rc ? rc : rt;
 }
 
@@ -539,6 +543,11 @@ int fsig_match_noalloc(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32
   }
   if (rc == FSIG_OK)
     rc = match_impl(c, g, k, qlabels, qoff, qadj, qsig, alg, mode, max_emb, count_out, emb_out, emb_cap, nullptr);
+  if (rc != FSIG_EHIP) {  // the counters at the scratch array's end are this call's only
+    const std::string err = c->err;
+    if (fetch_stats(c) != FSIG_OK) rc = FSIG_EHIP;
+    else c->err = err;
+  }
   if (rc == FSIG_ENOMEM) c->err = "noalloc: the static scratch is exhausted (" + c->err + ")";
   c->arena = saved_arena;
   c->d_counters = saved_counters;
@@ -606,12 +615,20 @@ int fsig_set_profiling(fsig_ctx* c, int on) {
 
 int fsig_stats_reset(fsig_ctx* c) {
   if (!c) return FSIG_EINVAL;
+  FSIG_HIP(c, hipSetDevice(c->device));
+  const int rc = fetch_stats(c);  // zeroes the device's part
+  if (rc) return rc;
   for (auto& s : c->kstat) s = KStat();
   return FSIG_OK;
 }
 
 int fsig_kernel_stats(const fsig_ctx* c, int fam, uint64_t* launches, double* ms, uint64_t* bytes, uint64_t* units) {
   if (!c || fam < 0 || fam >= FSIG_K_NUM) return FSIG_EINVAL;
+  // the device's part of the statistics stays there until somebody asks
+  fsig_ctx* m = const_cast<fsig_ctx*>(c);
+  FSIG_HIP(m, hipSetDevice(c->device));
+  const int rc = fetch_stats(m);
+  if (rc) return rc;
   const KStat& s = c->kstat[fam];
   if (launches) *launches = s.launches;
   if (ms) *ms = s.ms;

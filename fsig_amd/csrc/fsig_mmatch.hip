@@ -160,10 +160,14 @@ __global__ void k_scatter_pos(const uint32_t* __restrict__ cand, uint32_t n, uin
   for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) pos[cand[j]] = j;
 }
 
-__global__ void k_gather_u64(const uint64_t* __restrict__ src, const PairDesc* __restrict__ P, uint32_t np,
-                             uint64_t* __restrict__ out) {
+// out[i] = first list entry of pair i; out[np] = the number of list entries,
+// out[np + 1] = *entries: all that the host waits for, in one read.
+__global__ void k_pair_bases(const uint64_t* __restrict__ gscan, const PairDesc* __restrict__ P, uint32_t np,
+                             uint64_t rows, const uint64_t* __restrict__ entries, uint64_t* __restrict__ out) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < np) out[i] = src[P[i].flat];
+  if (i < np) out[i] = gscan[P[i].flat];
+  else if (i == np) out[i] = gscan[rows];
+  else if (i == np + 1) out[i] = *entries;
 }
 
 }  // namespace
@@ -506,26 +510,26 @@ int run_mmatch(fsig_ctx* c, const fsig_graph* g, QueryPlan& P, int mode, uint64_
     PairDesc* dP = (PairDesc*)A.alloc(sizeof(PairDesc) * np);
     uint32_t* cnt = (uint32_t*)A.alloc(4ull * flat);
     uint64_t* gscan = (uint64_t*)A.alloc(8ull * (flat + 1));
-    uint64_t* pbase = (uint64_t*)A.alloc(8ull * (np + 1));
+    uint64_t* pbase = (uint64_t*)A.alloc(8ull * (np + 2));
     if (!dP || !cnt || !gscan || !pbase) return set_err(c, FSIG_ENOMEM, "cedge: arena exhausted");
     FSIG_HIP(c, hipMemcpyAsync(dP, pairs.data(), sizeof(PairDesc) * np, hipMemcpyHostToDevice, c->stream));
     if ((rc = row_count(c, RG, dP, np, flat, g->d_off, g->d_adj, cnt))) return rc;
     SegRows segs;  // hub rows, one wavefront per segment
-    if ((rc = seg_prepare(c, dP, np, flat, g->d_off, cnt, segs))) return rc;
+    if ((rc = seg_prepare(c, dP, np, flat, g->d_off, cnt, g->max_degree > kHubDeg, segs))) return rc;
     if ((rc = seg_count(c, dP, np, flat, g->d_off, g->d_adj, cnt, segs))) return rc;
     FSIG_HIP(c, hipGetLastError());
     if ((rc = scan_u32_to_u64(c, cnt, gscan, flat))) return rc;
-    uint64_t total_edges;
-    if ((rc = read_u64(c, gscan + flat, &total_edges, 1))) return rc;
+    k_pair_bases<<<(np + 2 + 255) / 256, 256, 0, c->stream>>>(gscan, dP, np, flat, segs.segbase + flat + 1, pbase);
+    FSIG_HIP(c, hipGetLastError());
+    std::vector<uint64_t> hb(np + 2);
+    if ((rc = read_u64(c, pbase, hb.data(), np + 2))) return rc;
+    const uint64_t total_edges = hb[np];
+    segs.entries = hb[np + 1];
     uint32_t* lst_all = (uint32_t*)A.alloc(4ull * std::max<uint64_t>(total_edges, 1));
     if (!lst_all) return set_err(c, FSIG_ENOMEM, "cedge: arena exhausted for lists");
     if ((rc = row_fill(c, RG, dP, np, flat, g->d_off, g->d_adj, gscan, lst_all))) return rc;
     if ((rc = seg_fill(c, dP, np, flat, g->d_off, g->d_adj, gscan, lst_all, segs))) return rc;
-    k_gather_u64<<<(np + 255) / 256, 256, 0, c->stream>>>(gscan, dP, np, pbase);
     FSIG_HIP(c, hipGetLastError());
-    std::vector<uint64_t> hb(np);
-    for (uint32_t i = 0; i < np; i += 4096)
-      if ((rc = read_u64(c, pbase + i, hb.data() + i, std::min<uint32_t>(4096, np - i)))) return rc;
     for (uint32_t o = 0; o < 3; o++)
       for (uint32_t a = 0; a < nc; a++)
         for (uint32_t b = 0; b < nc; b++)

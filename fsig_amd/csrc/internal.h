@@ -179,7 +179,7 @@ int set_err(fsig_ctx* c, int code, const std::string& msg);
 
 // Timing of one kernel family around a launch sequence: with profiling on,
 // an event pair brackets the launches on the context stream; the pairs are
-// resolved by resolve_timings() once the stream has drained.
+// resolved by resolve_events() once the stream has drained.
 struct KTimer {
   fsig_ctx* c;
   int fam;
@@ -207,9 +207,11 @@ struct KTimer {
     if (slot != ~(size_t)0) (void)hipEventRecord(c->timed[slot].b, c->stream);
   }
 };
-// Adds the recorded event intervals and the device-side family counters into
-// the context statistics; the stream must be idle.
-int resolve_timings(fsig_ctx* c);
+// Adds the recorded event intervals into the context statistics; the stream
+// must be idle.
+int resolve_events(fsig_ctx* c);
+// Moves the device-side family counters into the context statistics.
+int fetch_stats(fsig_ctx* c);
 static_assert(2 * FSIG_K_NUM <= (int)kStripeWords, "the families' counters fit one copy");
 constexpr size_t kCounterWords = 2 * kStripes * kStripeWords;
 inline unsigned long long* family_counters(fsig_ctx* c, int fam) {

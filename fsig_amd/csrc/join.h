@@ -112,6 +112,7 @@ struct JoinIO {
   uint64_t out_lo, out_hi;    // write pass: children [out_lo, out_hi) are written, at out_lo -> out[0]
   unsigned long long* total;  // count pass: += children (may be null)
   unsigned long long* stats;  // [0] += algorithmic bytes, [1] += units (rows or children)
+  const unsigned long long* win;  // write pass, may be null: of the row range, only [win[0], win[1])
 };
 
 // Candidate-edge CSR lists (alg 1): list i of row value x (a candidate index of
@@ -227,7 +228,12 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_join(JoinLevel L, Src S, JoinIO 
   const uint64_t ngroups = (uint64_t)gridDim.x * GPB;
   unsigned long long my_children = 0, my_bytes = 0, my_rows = 0;
 
-  for (uint64_t r = io.row_lo + (uint64_t)xcd_block() * GPB + gw; r < io.row_hi; r += ngroups) {
+  uint64_t row_lo = io.row_lo, row_hi = io.row_hi;
+  if (WRITE && io.win) {
+    row_lo = max(row_lo, (uint64_t)io.win[0]);
+    row_hi = min(row_hi, (uint64_t)io.win[1]);
+  }
+  for (uint64_t r = row_lo + (uint64_t)xcd_block() * GPB + gw; r < row_hi; r += ngroups) {
     uint32_t rv[NR];
     const uint32_t* row = io.rows + r * L.p;
 #pragma unroll
@@ -813,7 +819,7 @@ struct TailIO {
   const uint32_t* rows;
   uint64_t nrows;
   uint32_t* cnt;              // per row: children of a deferred row, else 0
-  unsigned long long* res;    // [0] += leaves, [1] += children of counted rows
+  unsigned long long* res;    // [0] += leaves, [1] += children of counted rows, [2] += of deferred rows
   unsigned long long* stats;  // [0] += algorithmic bytes, [1] += parent rows
   uint32_t tile_words;        // shared-intersection tile per group (dynamic LDS)
   uint32_t kids_are_shared;   // the child level intersects the leaf's shared lists
@@ -851,7 +857,8 @@ k_join_tail(JoinLevel L1, CandEdgeSrc S1, JoinLevel L2, CandEdgeSrc S2, TailIO i
                                   KIND == kTailBoth && io.kids_are_shared);
     if (gl == 0) {
       io.cnt[r] = defer ? (uint32_t)kids : 0u;
-      if (!defer) my_kids += kids;
+      if (defer) atomicAdd(io.res + 2 + (blockIdx.x & (kStripes - 1)) * kStripeWords, (unsigned long long)kids);  // rare
+      else my_kids += kids;
       my_rows += 1;
     }
   }
@@ -1153,30 +1160,34 @@ inline int launch_join_tail_chain(fsig_ctx* c, uint32_t G, const JoinLevel& L1, 
 }
 
 // Parent rows of the child window [lo, hi): out[0] = last r with off[r] <= lo,
-// out[1] = first r with off[r] >= hi (off has nrows+1 entries).
+// out[1] = first r with off[r] >= hi (off has nrows+1 entries).  The write
+// pass reads them on the device.  One wavefront each, 64 probes a step: 3
+// dependent loads find a row among 2^18 where one lane's binary search takes
+// 18 (5..15 us a window).
 static __global__ void k_window_rows(const uint64_t* __restrict__ off, uint64_t nrows, uint64_t lo, uint64_t hi,
                                      unsigned long long* __restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+  // Entries [0, a) lie below the answer, entry b (if there is one) does not.
+  // The last entries of `parts` parts lie below it, so a moves past those
+  // parts, and stays at most b: the next part ends at na + step - 1 >= na.
+  // (Taking the smaller of the two instead of na itself was compiled to a
+  // select on the comparison before it.)
   uint64_t a = 0, b = nrows + 1;
   while (a < b) {
-    const uint64_t m = (a + b) >> 1;
-    if (off[m] <= lo) a = m + 1; else b = m;
+    const uint64_t step = (b - a + 63) / 64;
+    const uint64_t m = a + (lane + 1) * step - 1;  // last entry of the lane's part of [a, b)
+    const bool below = m < b && (w == 0 ? off[m] <= lo : off[m] < hi);
+    a += (uint64_t)__popcll(__ballot(below)) * step;
+    b = min(b, a + step - 1);
   }
-  out[0] = a - 1;
-  a = 0;
-  b = nrows + 1;
-  while (a < b) {
-    const uint64_t m = (a + b) >> 1;
-    if (off[m] < hi) a = m + 1; else b = m;
-  }
-  out[1] = a > nrows ? nrows : a;
+  if (lane == 0) out[w] = w == 0 ? a - 1 : min(a, nrows);
 }
 
 // Host launcher for the join kernel, dispatching on G.
 template <int MODE, class Src>
 int launch_join(fsig_ctx* c, uint32_t G, const JoinLevel& L, const Src& S, const JoinIO& io,
-                const DigestArg<MODE>& D = DigestArg<MODE>()) {
-  const uint64_t nrows = io.row_hi - io.row_lo;
+                const DigestArg<MODE>& D = DigestArg<MODE>(), uint64_t span = ~0ull) {
+  const uint64_t nrows = std::min(span, io.row_hi - io.row_lo);  // (groups stride over the rest)
   if (nrows == 0) return FSIG_OK;
   const uint64_t gpb = FSIG_BLOCK / G;
   uint64_t blocks = (nrows + gpb - 1) / gpb;
@@ -1334,7 +1345,12 @@ class JoinDriver {
       if (fused) {
         // rows whose leaves the tail counts get 0 children; deferred rows
         // keep theirs and go through the write pass and the last level
-        if ((rc = count_tail(rows, R, cnt, L, S, pv_.level(p + 1), pv_.src(p + 1)))) return rc;
+        uint64_t deferred = 0;
+        if ((rc = count_tail(rows, R, cnt, L, S, pv_.level(p + 1), pv_.src(p + 1), deferred))) return rc;
+        if (deferred == 0) {  // the usual case: nothing to scan, nothing to read back
+          c_->arena.release(mk);
+          return FSIG_OK;
+        }
       }
     }
     if (!fused) {
@@ -1384,20 +1400,20 @@ class JoinDriver {
         window_[p] = std::min(window_[p] * 2, kGrowMax);
         wsize = std::min(std::min(cap, window_[p]), need_rows(p + 1));
       }
-      uint64_t win[2] = {0, R};
-      if (split) {  // parent rows of this window, found on the device
-        k_window_rows<<<1, 64, 0, c_->stream>>>(off, R, lo, hi, dwin);
+      if (split) {  // parent rows of this window, found and used on the device
+        k_window_rows<<<1, 128, 0, c_->stream>>>(off, R, lo, hi, dwin);
         FSIG_HIP(c_, hipGetLastError());
-        if ((rc = read_u64(c_, dwin, win, 2))) return rc;
       }
+      // rows to launch for: those with children are at most hi - lo
+      const uint64_t span = split ? std::min(R, hi - lo) : R;
       const size_t m2 = c_->arena.mark();
       uint32_t* child = (uint32_t*)c_->arena.alloc(4ull * (p + 1) * (hi - lo));
       if (!child) return set_err(c_, FSIG_ENOMEM, "join: arena exhausted for a window");
-      JoinIO io{rows, win[0], win[1], nullptr, off, child, lo, hi, nullptr,
-                family_counters(c_, FSIG_K_JOIN_WRITE)};
+      JoinIO io{rows, 0, R, nullptr, off, child, lo, hi, nullptr,
+                family_counters(c_, FSIG_K_JOIN_WRITE), dwin};
       {
         KTimer t(c_, FSIG_K_JOIN_WRITE);
-        if ((rc = launch_join<kJoinWrite>(c_, widen_lanes(c_, G_, win[1] - win[0], 64), L, S, io))) return rc;
+        if ((rc = launch_join<kJoinWrite>(c_, widen_lanes(c_, G_, span, 64), L, S, io, {}, span))) return rc;
         t.done(0, 0);
       }
       if ((rc = expand(p + 1, child, hi - lo))) return rc;
@@ -1412,7 +1428,7 @@ class JoinDriver {
   // are added to the total and their children count towards the work limit;
   // deferred rows keep their children in cnt.
   int count_tail(const uint32_t* rows, uint64_t R, uint32_t* cnt, const JoinLevel& L1, const CandEdgeSrc& S1,
-                 const JoinLevel& L2, const CandEdgeSrc& S2) {
+                 const JoinLevel& L2, const CandEdgeSrc& S2, uint64_t& deferred) {
     unsigned long long* res = c_->d_counters;
     int rc = clear_results(c_);
     if (rc) return rc;
@@ -1435,8 +1451,9 @@ class JoinDriver {
                        : launch_join_tail(c_, G, L1, S1, L2, S2, io);
     if (rc) return rc;
     t.done(0, 0);
-    uint64_t h[2];
-    if ((rc = read_striped(c_, res, h, 2))) return rc;
+    uint64_t h[3];
+    if ((rc = read_striped(c_, res, h, 3))) return rc;
+    deferred = h[2];
     rows_ += h[1];
     const uint64_t limit = c_->work_limit;
     if (limit && rows_ > limit) return set_err(c_, FSIG_ELIMIT, "join: work limit exceeded");
