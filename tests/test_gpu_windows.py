@@ -23,7 +23,7 @@ def test_bounded_windows(gpu_ctx, n, m, lanes):
     try:
         gpu_ctx.set_tune(lanes_per_row=lanes)
         total = F.match(dg, q, F.ALG_MMATCH, F.MODE_COUNT).count
-        want, _ = O.match(q.labels, q.adjm(), off, adj, lab, threads=8, limit=30_000_000)
+        want, _ = O.match(q.labels, q.adjm(), off, adj, lab, threads=8, limit=1 << 30)
         assert total == want
         for alg in (F.ALG_MMATCH, F.ALG_GSI):
             for b in (1, 63, 511, 512, 513, 1025, 4096, 40001, 300007):
