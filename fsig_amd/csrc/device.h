@@ -26,6 +26,14 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
   return v;
 }
 
+// Flag of a host mailbox (pinned coherent memory): the words written before
+// it, by this thread or by a block that has met at a barrier after its own
+// system fences, are visible to a host that reads `seq` from it.
+__device__ __forceinline__ void mail_flag(unsigned long long* flag, unsigned long long seq) {
+  __threadfence_system();
+  __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Sums into striped counters (kStripes).  Additions of 64-bit words to one
 // address take 12..13 ns each, one after another, however many compute units
 // send them: with one address and an addition per wavefront and counter, the

@@ -1722,9 +1722,8 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
       if ((rc = seg_count(c, dP, np, pflat, g->d_off, g->d_adj, cnt, segs, ch_seg[j], ch_seg[j + 1]))) return rc;
     }
     FSIG_HIP(c, hipGetLastError());
-    if ((rc = scan_u32_to_u64(c, cnt, gscan, pflat))) return rc;
     uint64_t total_edges;
-    if ((rc = read_u64(c, gscan + pflat, &total_edges, 1))) return rc;
+    if ((rc = scan_u32_to_u64(c, cnt, gscan, pflat, &total_edges))) return rc;
     lst_all = (uint32_t*)A.alloc(4ull * std::max<uint64_t>(total_edges, 1));
     if (!lst_all) return set_err(c, FSIG_ENOMEM, "batch: arena exhausted for candidate lists");
     for (size_t j = 0; j < nch; j++) {
@@ -1967,8 +1966,7 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
     for (uint32_t j = 0; j < nl; j++)
       if (cut[j] != ~0ull && cut[j] != 0 && first[j] < qb[j + 1])
         cut_rows[live[j]].push_back(CutRows{p, rows + first[j] * p, qb[j + 1] - first[j]});
-    if ((rc2 = scan_u32_to_u64(c, cnt, off, R))) return rc2;
-    return read_u64(c, off + R, &T, 1);
+    return scan_u32_to_u64(c, cnt, off, R, &T);
   };
   // The subtrees of the cut rows of every beamed query that ended below its
   // bound, counted by the bounded depth-first driver (bound: what the beam
@@ -2042,9 +2040,8 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
       std::vector<MLevel> ml(nl);
       uint64_t prev_bytes = 0;  // debug timing: device byte counter before the level
       auto level_bytes = [&]() -> uint64_t {
-        uint64_t w[2 * FSIG_K_BATCH + 1] = {0};
-        (void)read_striped(c, c->d_counters + kStripes * kStripeWords, w, 2 * FSIG_K_BATCH + 1);
-        return w[2 * FSIG_K_BATCH];
+        (void)fetch_stats(c);
+        return c->kstat[FSIG_K_BATCH].alg_bytes;
       };
       if (clk.on) prev_bytes = level_bytes();
       // one launch per lane-count group over its row range of the level
@@ -2093,9 +2090,8 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
         int rc2 = launch(false, p, cnt, off, nullptr);
         if (rc2) { A.release(mk); return rc2; }
         if (!any_more) break;
-        if ((rc2 = scan_u32_to_u64(c, cnt, off, R))) { A.release(mk); return rc2; }
         uint64_t T;
-        if ((rc2 = read_u64(c, off + R, &T, 1))) { A.release(mk); return rc2; }
+        if ((rc2 = scan_u32_to_u64(c, cnt, off, R, &T))) { A.release(mk); return rc2; }
         if (any_bound && (rc2 = settle_bounded(p, rows, cnt, off, R, dqb, dqb2, qb, live, T))) {
           A.release(mk);
           return rc2;

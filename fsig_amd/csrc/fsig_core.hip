@@ -1,6 +1,7 @@
 // libfsig_hip.so: context, arena, resident graph, device scan and the C ABI
 // entry points of include/fsig.h.
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <mutex>
 
@@ -32,7 +33,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_scan_tile_sums(const uint32_t* _
 }
 
 __global__ void __launch_bounds__(FSIG_BLOCK) k_scan_tile_offsets(uint64_t* __restrict__ sums, uint64_t ntiles,
-                                                                  uint64_t* __restrict__ total_out) {
+                                                                  uint64_t* __restrict__ total_out, Mail mail) {
   __shared__ uint64_t lds[4];
   uint64_t carry = 0;
   for (uint64_t b = 0; b < ntiles; b += FSIG_BLOCK) {
@@ -43,7 +44,46 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_scan_tile_offsets(uint64_t* __re
     if (i < ntiles) sums[i] = carry + ex;
     carry += tot;
   }
-  if (threadIdx.x == 0) *total_out = carry;
+  if (threadIdx.x == 0) {
+    *total_out = carry;
+    if (mail.flag) {
+      mail.words[0] = carry;
+      mail_flag(mail.flag, mail.seq);
+    }
+  }
+}
+
+// The whole scan in one workgroup for few items: 3 launches of 3 us each and
+// the gaps between them become one.
+__global__ void __launch_bounds__(FSIG_BLOCK) k_scan_small(const uint32_t* __restrict__ in, uint32_t n,
+                                                           uint64_t* __restrict__ out, Mail mail) {
+  __shared__ uint64_t lds[4];
+  uint64_t carry = 0;
+  for (uint32_t b = 0; b < n; b += kTile) {
+    const uint32_t base = b + threadIdx.x * 4;
+    uint32_t v[4];
+    uint64_t s = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      v[j] = base + j < n ? in[base + j] : 0;
+      s += v[j];
+    }
+    uint64_t tot;
+    uint64_t ex = block_exclusive_scan(s, lds, tot) + carry;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if (base + j < n) out[base + j] = ex;
+      ex += v[j];
+    }
+    carry += tot;
+  }
+  if (threadIdx.x == 0) {
+    out[n] = carry;
+    if (mail.flag) {
+      mail.words[0] = carry;
+      mail_flag(mail.flag, mail.seq);
+    }
+  }
 }
 
 __global__ void __launch_bounds__(FSIG_BLOCK) k_scan_tiles(const uint32_t* __restrict__ in, uint64_t n,
@@ -73,6 +113,37 @@ __global__ void k_fill_words(uint32_t* __restrict__ p, uint32_t n) {
   for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
 }
 
+// Sends `count` device words by mail (one block).
+__global__ void __launch_bounds__(FSIG_BLOCK) k_post(const unsigned long long* __restrict__ src, uint32_t count,
+                                                     Mail mail) {
+  for (uint32_t i = threadIdx.x; i < count; i += FSIG_BLOCK) mail.words[i] = src[i];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) mail_flag(mail.flag, mail.seq);
+}
+
+// Sends the sums of striped counters by mail and zeroes them (one block).
+__global__ void __launch_bounds__(FSIG_BLOCK) k_take_striped(unsigned long long* __restrict__ dev, Mail mail) {
+  constexpr uint32_t kParts = FSIG_BLOCK / kStripeWords;
+  __shared__ unsigned long long part[kParts][kStripeWords];
+  const uint32_t w = threadIdx.x % kStripeWords, q = threadIdx.x / kStripeWords;
+  unsigned long long s = 0;
+  for (uint32_t j = q; j < kStripes; j += kParts) {
+    s += dev[j * kStripeWords + w];
+    dev[j * kStripeWords + w] = 0;
+  }
+  part[q][w] = s;
+  __syncthreads();
+  if (threadIdx.x < kStripeWords) {
+    s = 0;
+    for (uint32_t j = 0; j < kParts; j++) s += part[j][threadIdx.x];
+    mail.words[threadIdx.x] = s;
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) mail_flag(mail.flag, mail.seq);
+}
+
 // Plain copy, 16 bytes per thread per step (the STREAM "copy" kernel).
 __global__ void __launch_bounds__(FSIG_BLOCK) k_stream_copy(const uint4* __restrict__ src, uint4* __restrict__ dst,
                                                             uint64_t n) {
@@ -82,22 +153,30 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_stream_copy(const uint4* __restr
 
 }  // namespace
 
-int scan_u32_to_u64(fsig_ctx* c, const uint32_t* in, uint64_t* out, uint64_t n) {
+// One workgroup scans up to this many items (four steps).
+constexpr uint64_t kScanSmall = 4 * kTile;
+
+int scan_u32_to_u64(fsig_ctx* c, const uint32_t* in, uint64_t* out, uint64_t n, uint64_t* total) {
   KTimer t(c, FSIG_K_SCAN);
   const uint64_t ntiles = (n + kTile - 1) / kTile;
   size_t mk = c->arena.mark();
   uint64_t* sums = (uint64_t*)c->arena.alloc(sizeof(uint64_t) * std::max<uint64_t>(ntiles, 1));
   if (!sums) return set_err(c, FSIG_ENOMEM, "scan: arena exhausted");
-  if (ntiles > 0) {
+  const Mail mail = total ? mail_next(c) : Mail{nullptr, nullptr, 0};
+  if (n <= kScanSmall) {
+    k_scan_small<<<1, FSIG_BLOCK, 0, c->stream>>>(in, (uint32_t)n, out, mail);
+  } else {
     k_scan_tile_sums<<<(uint32_t)ntiles, FSIG_BLOCK, 0, c->stream>>>(in, n, sums);
-  }
-  k_scan_tile_offsets<<<1, FSIG_BLOCK, 0, c->stream>>>(sums, ntiles, out + n);
-  if (ntiles > 0) {
+    k_scan_tile_offsets<<<1, FSIG_BLOCK, 0, c->stream>>>(sums, ntiles, out + n, mail);
     k_scan_tiles<<<(uint32_t)ntiles, FSIG_BLOCK, 0, c->stream>>>(in, n, sums, out);
   }
   FSIG_HIP(c, hipGetLastError());
   c->arena.release(mk);
   t.done(n * 4 + n * 8 + 8, n);
+  if (!total) return FSIG_OK;
+  const int rc = mail_wait(c, mail);
+  if (rc) return rc;
+  *total = mail.words[0];
   return FSIG_OK;
 }
 
@@ -112,36 +191,59 @@ int resolve_events(fsig_ctx* c) {
 }
 
 int fetch_stats(fsig_ctx* c) {
-  constexpr size_t kWords = kStripes * kStripeWords;
-  uint64_t fam[kWords];
-  int rc = read_u64(c, c->d_counters + kWords, fam, kWords);
+  uint64_t fam[2 * FSIG_K_NUM];
+  const int rc = take_striped(c, family_counters(c, 0), fam, 2 * FSIG_K_NUM);
   if (rc) return rc;
-  for (uint32_t s = 0; s < kStripes; s++)
-    for (int f = 0; f < FSIG_K_NUM; f++) {
-      c->kstat[f].alg_bytes += fam[s * kStripeWords + 2 * f];
-      c->kstat[f].units += fam[s * kStripeWords + 2 * f + 1];
+  for (int f = 0; f < FSIG_K_NUM; f++) {
+    c->kstat[f].alg_bytes += fam[2 * f];
+    c->kstat[f].units += fam[2 * f + 1];
+  }
+  return FSIG_OK;
+}
+
+Mail mail_next(fsig_ctx* c) { return Mail{c->h_pinned, c->h_pinned + kPinnedWords, ++c->mail_seq}; }
+
+// The flag is polled for a millisecond, beyond which the wake-up of a
+// blocking wait no longer matters; that wait also ends, with its error, when
+// a kernel of the stream has failed and no flag will come.
+int mail_wait(fsig_ctx* c, const Mail& m) {
+  auto here = [&] { return __atomic_load_n(m.flag, __ATOMIC_ACQUIRE) == m.seq; };
+  const auto t0 = std::chrono::steady_clock::now();
+  for (;;) {
+    for (int i = 0; i < 64; i++) {
+      if (here()) return FSIG_OK;
+      __builtin_ia32_pause();
     }
-  FSIG_HIP(c, hipMemsetAsync(c->d_counters + kWords, 0, 8 * kWords, c->stream));
-  return FSIG_OK;
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(1)) break;
+  }
+  FSIG_HIP(c, hipStreamSynchronize(c->stream));
+  return here() ? FSIG_OK : set_err(c, FSIG_EHIP, "a kernel of this context ended without its result");
 }
 
-int clear_results(fsig_ctx* c) {
-  FSIG_HIP(c, hipMemsetAsync(c->d_counters, 0, 8 * kStripes * kStripeWords, c->stream));
-  return FSIG_OK;
-}
-
-int read_striped(fsig_ctx* c, const unsigned long long* dev, uint64_t* host, uint32_t n) {
-  uint64_t all[kStripes * kStripeWords];
-  const int rc = read_u64(c, dev, all, kStripes * kStripeWords);
+int take_striped(fsig_ctx* c, unsigned long long* dev, uint64_t* host, uint32_t n) {
+  const Mail m = mail_next(c);
+  k_take_striped<<<1, FSIG_BLOCK, 0, c->stream>>>(dev, m);
+  FSIG_HIP(c, hipGetLastError());
+  const int rc = mail_wait(c, m);
   if (rc) return rc;
-  for (uint32_t i = 0; i < n; i++) host[i] = 0;
-  for (uint32_t s = 0; s < kStripes; s++)
-    for (uint32_t i = 0; i < n; i++) host[i] += all[s * kStripeWords + i];
+  for (uint32_t i = 0; i < n; i++) host[i] = m.words[i];
   return FSIG_OK;
 }
 
 int read_u64(fsig_ctx* c, const void* dev, uint64_t* host, size_t count) {
   if (count > kPinnedWords) return set_err(c, FSIG_EINVAL, "read_u64: too many words");
+  // A blocking copy of a few words costs a copy kernel, a completion signal
+  // and the host's wake-up, some 15 us of an idle device; the posting kernel
+  // and the poll cost about 6.
+  if (count <= kMailWords) {
+    const Mail m = mail_next(c);
+    k_post<<<1, FSIG_BLOCK, 0, c->stream>>>((const unsigned long long*)dev, (uint32_t)count, m);
+    FSIG_HIP(c, hipGetLastError());
+    const int rc = mail_wait(c, m);
+    if (rc) return rc;
+    std::memcpy(host, m.words, count * 8);
+    return FSIG_OK;
+  }
   FSIG_HIP(c, hipMemcpyAsync(c->h_pinned, dev, count * 8, hipMemcpyDeviceToHost, c->stream));
   FSIG_HIP(c, hipStreamSynchronize(c->stream));
   std::memcpy(host, c->h_pinned, count * 8);
@@ -196,7 +298,8 @@ int fsig_ctx_create(int device, uint64_t budget, fsig_ctx** out) {
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreate(&c->ev_a) != hipSuccess || hipEventCreate(&c->ev_b) != hipSuccess ||
       hipMalloc((void**)&c->d_counters, kCounterWords * sizeof(unsigned long long)) != hipSuccess ||
-      hipHostMalloc((void**)&c->h_pinned, kPinnedWords * 8, hipHostMallocDefault) != hipSuccess) {
+      hipHostMalloc((void**)&c->h_pinned, (kPinnedWords + 8) * 8, hipHostMallocMapped | hipHostMallocCoherent) !=
+          hipSuccess) {
     fsig_ctx_destroy(c);
     return FSIG_EHIP;
   }
@@ -205,7 +308,9 @@ int fsig_ctx_create(int device, uint64_t budget, fsig_ctx** out) {
     return FSIG_ENOMEM;
   }
   c->arena.cap = budget;
-  if (hipMemset(c->d_counters, 0, kCounterWords * sizeof(unsigned long long)) != hipSuccess) {
+  c->h_pinned[kPinnedWords] = 0;
+  if (hipMemsetAsync(c->d_counters, 0, kCounterWords * sizeof(unsigned long long), c->stream) != hipSuccess ||
+      hipStreamSynchronize(c->stream) != hipSuccess) {
     fsig_ctx_destroy(c);
     return FSIG_EHIP;
   }
@@ -446,11 +551,16 @@ static int match_impl(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
     *count_out = orbits > UINT64_MAX / P.aut ? UINT64_MAX : orbits * P.aut;
     if (max_emb) *count_out = std::min(*count_out, max_emb);
   }
-  if (rc == FSIG_OK && acc) rc = read_striped(c, acc, digest_out, 2);
+  if (rc == FSIG_OK && acc) rc = take_striped(c, acc, digest_out, 2);
   c->last_peak = c->arena.peak - mk;
   c->arena.release(mk);
-  hipError_t e = hipStreamSynchronize(c->stream);
-  if (e != hipSuccess) return set_err(c, FSIG_EHIP, std::string("match: ") + hipGetErrorString(e));
+  // A count that went well ended with a read by mail, behind all kernels it
+  // depends on (at most the scan of a level without children is left); the
+  // end of the stream itself is waited for otherwise, and for event timings.
+  if (rc || mode != FSIG_MODE_COUNT || digest_out || c->timed_used) {
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return set_err(c, FSIG_EHIP, std::string("match: ") + hipGetErrorString(e));
+  }
   int rt = resolve_events(c);
   return rc ? rc : rt;
 }

@@ -164,7 +164,6 @@ struct GsiProvider {
     KTimer t(c, FSIG_K_JOIN_COUNT);
     if ((rc = launch_join<kJoinCount>(c, widen_lanes(c, G, csize[a], 64), one, S, io))) return rc;
     k_scatter_counts<<<grid_for(c, csize[a], FSIG_BLOCK), FSIG_BLOCK, 0, c->stream>>>(cand[a], csize[a], cnt, leaves);
-    if ((rc = clear_results(c))) return rc;
     uint64_t blocks = std::min<uint64_t>((R + FSIG_BLOCK - 1) / FSIG_BLOCK, (uint64_t)c->num_cus * 16);
     if (blocks >= 64) blocks &= ~7ull;
     k_leaf_sum<<<(uint32_t)blocks, FSIG_BLOCK, 0, c->stream>>>(L, rows, R, leaves, mask, S.wbit, g->d_off, g->d_adj,
@@ -173,7 +172,7 @@ struct GsiProvider {
     t.done(0, 0);
     c->arena.release(mk);
     counted = true;
-    return read_striped(c, c->d_counters, &sum, 1);
+    return take_striped(c, c->d_counters, &sum, 1);
   }
   PcsrSrc src(uint32_t p) const {
     PcsrSrc S;

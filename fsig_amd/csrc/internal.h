@@ -13,6 +13,8 @@
 
 #define MAXQ 32
 constexpr size_t kPinnedWords = 65536;
+// Reads of up to this many words go through the mailbox (fsig_ctx::h_pinned).
+constexpr size_t kMailWords = 1024;
 #define FSIG_INVALID 0xffffffffu
 // Device counters are kept in kStripes copies of kStripeWords words (one
 // cache line) each: a block adds to the copy of its number (block_add) and
@@ -83,7 +85,10 @@ struct fsig_ctx {
   // kernel family f (word 2f algorithmic bytes, 2f+1 units); see block_add.
   // Host staging is pinned.
   unsigned long long* d_counters = nullptr;
-  unsigned long long* h_pinned = nullptr;  // kPinnedWords words of pinned staging
+  // kPinnedWords words of pinned staging, then the mailbox flag: a kernel
+  // writes words here and then mail_seq to the flag, and the host polls it
+  unsigned long long* h_pinned = nullptr;
+  unsigned long long mail_seq = 0;
   int num_cus = 256;
   // choice of the batched engine's autotuner on its last batch
   uint64_t work_limit = 0;  // max intermediate rows per fsig_match (0 = none)
@@ -217,19 +222,33 @@ constexpr size_t kCounterWords = 2 * kStripes * kStripeWords;
 inline unsigned long long* family_counters(fsig_ctx* c, int fam) {
   return c->d_counters + kStripes * kStripeWords + 2 * fam;
 }
-// Zeroes the per-launch results (on the stream) / reads the sums of the
-// first n words of striped counters.
-int clear_results(fsig_ctx* c);
-int read_striped(fsig_ctx* c, const unsigned long long* dev, uint64_t* host, uint32_t n);
+// Reads the sums of the first n words of striped counters and zeroes them
+// (so every launch finds its results at zero).
+int take_striped(fsig_ctx* c, unsigned long long* dev, uint64_t* host, uint32_t n);
 // Refinement passes: the tuned cap, else 2 (one query or a batch).  After
 // the neighbour-label filter the second pass still pays for itself on large
 // graphs (smaller candidate edges and joins); later ones remove a few
 // candidates at the price of a full pass.
 inline uint32_t refine_passes(const fsig_ctx* c) { return c->tune.refine_passes ? c->tune.refine_passes : 2u; }
 
+// The context's mailbox: a kernel of its stream writes its words to
+// Mail::words and then, with mail_flag(flag, seq), the flag; mail_wait
+// returns once the flag has arrived.  One mail is on its way at a time (a
+// context is used by one thread at a time) and its words are read before the
+// next is sent.  The kernels before the sender have then finished; later ones
+// may still run.
+struct Mail {
+  unsigned long long* words;
+  unsigned long long* flag;
+  unsigned long long seq;
+};
+Mail mail_next(fsig_ctx* c);
+int mail_wait(fsig_ctx* c, const Mail& m);
+
 // Device-wide exclusive scan of n u32 counts into out[0..n] (u64, out[n] is
-// the total).  Temporary storage comes from the arena.
-int scan_u32_to_u64(fsig_ctx* c, const uint32_t* in, uint64_t* out, uint64_t n);
+// the total).  Temporary storage comes from the arena.  With `total` the host
+// waits for the total (not for the scan's last pass).
+int scan_u32_to_u64(fsig_ctx* c, const uint32_t* in, uint64_t* out, uint64_t n, uint64_t* total = nullptr);
 
 // Reads `count` u64 words from device to host through the pinned staging area.
 int read_u64(fsig_ctx* c, const void* dev, uint64_t* host, size_t count);

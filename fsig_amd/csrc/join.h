@@ -1298,7 +1298,7 @@ class JoinDriver {
     const JoinLevel L = pv_.level(p);
     const Src S = pv_.src(p);
     const bool last = p + 1 == k_;
-    unsigned long long* res = c_->d_counters;  // [0] children of this launch
+    unsigned long long* res = c_->d_counters;  // [0] children of this launch (zero between launches)
     int rc;
     bool fused = false;
     if constexpr (std::is_same<Src, CandEdgeSrc>::value)
@@ -1315,26 +1315,24 @@ class JoinDriver {
           return FSIG_OK;
         }
       }
-      if ((rc = clear_results(c_))) return rc;
       JoinIO io{rows, 0, R, nullptr, nullptr, nullptr, 0, 0, res, family_counters(c_, FSIG_K_JOIN_COUNT)};
       KTimer t(c_, FSIG_K_JOIN_COUNT);
       if ((rc = launch_join<kJoinCount>(c_, widen_lanes(c_, G_, R, 64), L, S, io))) return rc;
       t.done(0, 0);
       uint64_t h;
-      if ((rc = read_striped(c_, res, &h, 1))) return rc;
+      if ((rc = take_striped(c_, res, &h, 1))) return rc;
       total_ += std::min(h, remaining());
       return FSIG_OK;
     }
     if (const DigestMap* D = last && sink_ && !bounded() ? sink_->digest() : nullptr) {
       // every child is an embedding and is only digested: no offsets, no
       // table, no second pass
-      if ((rc = clear_results(c_))) return rc;
       JoinIO io{rows, 0, R, nullptr, nullptr, nullptr, 0, 0, res, family_counters(c_, FSIG_K_JOIN_COUNT)};
       KTimer t(c_, FSIG_K_JOIN_COUNT);
       if ((rc = launch_join<kJoinDigest>(c_, widen_lanes(c_, G_, R, 64), L, S, io, *D))) return rc;
       t.done(0, 0);
       uint64_t h;
-      if ((rc = read_striped(c_, res, &h, 1))) return rc;
+      if ((rc = take_striped(c_, res, &h, 1))) return rc;
       total_ += h;
       return FSIG_OK;
     }
@@ -1359,9 +1357,8 @@ class JoinDriver {
       if ((rc = launch_join<kJoinCount>(c_, widen_lanes(c_, G_, R, 64), L, S, io))) return rc;
       t.done(0, 0);
     }
-    if ((rc = scan_u32_to_u64(c_, cnt, off, R))) return rc;
     uint64_t T;
-    if ((rc = read_u64(c_, off + R, &T, 1))) return rc;
+    if ((rc = scan_u32_to_u64(c_, cnt, off, R, &T))) return rc;
     if (T == 0) { c_->arena.release(mk); return FSIG_OK; }
     if (last) T = std::min(T, remaining());
     const uint64_t limit = c_->work_limit;
@@ -1430,8 +1427,6 @@ class JoinDriver {
   int count_tail(const uint32_t* rows, uint64_t R, uint32_t* cnt, const JoinLevel& L1, const CandEdgeSrc& S1,
                  const JoinLevel& L2, const CandEdgeSrc& S2, uint64_t& deferred) {
     unsigned long long* res = c_->d_counters;
-    int rc = clear_results(c_);
-    if (rc) return rc;
     ChainTail chain;
     const bool use_chain = chain_tail_applies(L1, L2) && pv_.chain_tail(L1.p, chain);
     // lanes per parent row: at least 8 where the shared intersection goes
@@ -1447,12 +1442,12 @@ class JoinDriver {
                     use_chain ? 0u : tail_tile_words(G, L2, c_->tune.lds_tile),
                     tail_kids_shared(L1, S1, L2, S2) ? 1u : 0u};
     KTimer t(c_, FSIG_K_JOIN_TAIL);
-    rc = use_chain ? launch_join_tail_chain(c_, G, L1, S1, L2, S2, chain, io)
+    int rc = use_chain ? launch_join_tail_chain(c_, G, L1, S1, L2, S2, chain, io)
                        : launch_join_tail(c_, G, L1, S1, L2, S2, io);
     if (rc) return rc;
     t.done(0, 0);
     uint64_t h[3];
-    if ((rc = read_striped(c_, res, h, 3))) return rc;
+    if ((rc = take_striped(c_, res, h, 3))) return rc;
     deferred = h[2];
     rows_ += h[1];
     const uint64_t limit = c_->work_limit;
