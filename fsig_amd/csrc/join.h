@@ -605,8 +605,8 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
   // the latency of those reads and of the row's own range lookups.  With
   // lists ordered by degree, the triangle on the 2^20-vertex, 8.75M-edge
   // R-MAT graph went from 27.7 to 7.1 ms and the 4-clique on the 2^18-vertex,
-  // 2.19M-edge one from 37.6 to 8.0 ms (one child at a time and binary
-  // searches, ordered by degree: 17.5 and 11.8 ms).
+  // 2.19M-edge one from 37.6 to 8.0 ms (6.0 and 6.2 ms now; one child at a
+  // time and binary searches, ordered by degree: 17.5 and 11.8 ms).
   uint32_t hsize = 0, hshift = 0;
   uint32_t* hset = sh.tile + isz;
   if (KIND == kTailBoth && !defer_row && 2 * isz > (uint32_t)G && tb1 - ta1 > 2) {
@@ -945,13 +945,17 @@ inline bool tail_kids_shared(const JoinLevel& L1, const CandEdgeSrc& S1, const J
 
 // Tile words per group the tail of L2 needs: only a leaf with both shared
 // lists (parent columns) and an own list (column p) intersects in LDS.
-// 16 KiB per block; twice that where lists ordered by degree are intersected,
-// whose few hundred entries then fit beside their hash set.
+// 16 KiB per block; 22 KiB where lists ordered by degree are intersected: a
+// wavefront's 1,408 words hold up to 384 entries beside their hash set (the
+// longest list has 446 on the 2^20-vertex R-MAT graph; longer ones are
+// searched), and six blocks fit a compute unit where 32 KiB let four.
+// Triangle on that graph / 4-clique on the 2^18-vertex one: 32 KiB 7.1 / 6.9
+// ms, 24 KiB 6.3 / 6.2, 22 KiB 6.0 / 6.2, 20 KiB 7.0 / 5.7, 16 KiB 7.4 / 6.0.
 inline uint32_t tail_tile_words(uint32_t G, const JoinLevel& L2, uint32_t cap) {
   bool shared = false, own = false;
   for (uint32_t i = 0; i < L2.nb; i++) (L2.bcol[i] == L2.p - 1 ? own : shared) = true;
   if (!shared || !own) return 0;
-  const uint32_t w = (L2.oriented ? 8192 : 4096) / (FSIG_BLOCK / G);
+  const uint32_t w = (L2.oriented ? 5632 : 4096) / (FSIG_BLOCK / G);
   return cap && cap < w ? cap : w;
 }
 
