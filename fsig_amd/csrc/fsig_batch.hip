@@ -1309,6 +1309,7 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
   std::vector<uint32_t> cls_base(nq + 1, 0);
   for (uint32_t i = 0; i < nq; i++) cls_base[i + 1] = cls_base[i] + plans[i].nclass;
   const uint32_t ncls = cls_base[nq];
+  if ((rc = begin_counters(c))) return rc;
   KTimer tf(c, FSIG_K_FILTER);
   uint32_t* masks = (uint32_t*)A.alloc(4ull * std::max<uint32_t>(n, 1) * nq);
   if (!masks) return set_err(c, FSIG_ENOMEM, "batch: arena exhausted for candidate masks");
@@ -2278,6 +2279,7 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
   std::vector<uint64_t> hc(nq);
   for (uint32_t i = 0; i < nq; i += kPinnedWords)
     if ((rc = read_u64(c, dcounts + i, hc.data() + i, std::min<size_t>(kPinnedWords, nq - i)))) return rc;
+  c->counters_open = false;
   clk.mark("lockstep join");
   if (clk.on) {
     uint32_t nbeamed = 0;

@@ -220,6 +220,15 @@ int mail_wait(fsig_ctx* c, const Mail& m) {
   return here() ? FSIG_OK : set_err(c, FSIG_EHIP, "a kernel of this context ended without its result");
 }
 
+int begin_counters(fsig_ctx* c) {
+  if (c->counters_open) {
+    k_fill_words<<<1, FSIG_BLOCK, 0, c->stream>>>((uint32_t*)c->d_counters, 2 * kStripes * kStripeWords);
+    FSIG_HIP(c, hipGetLastError());
+  }
+  c->counters_open = true;
+  return FSIG_OK;
+}
+
 int take_striped(fsig_ctx* c, unsigned long long* dev, uint64_t* host, uint32_t n) {
   const Mail m = mail_next(c);
   k_take_striped<<<1, FSIG_BLOCK, 0, c->stream>>>(dev, m);
@@ -517,6 +526,7 @@ static int match_impl(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
       if (c->keep_cand) c->cand_sets[0].assign(k, {}), c->cand_sets[1].assign(k, {});
       return FSIG_OK;
     }
+  if ((rc = begin_counters(c))) return rc;
   const size_t mk = c->arena.mark();
   c->arena.peak = mk;
   unsigned long long* acc = nullptr;
@@ -552,6 +562,7 @@ static int match_impl(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
     if (max_emb) *count_out = std::min(*count_out, max_emb);
   }
   if (rc == FSIG_OK && acc) rc = take_striped(c, acc, digest_out, 2);
+  if (rc == FSIG_OK) c->counters_open = false;
   c->last_peak = c->arena.peak - mk;
   c->arena.release(mk);
   // A count that went well ended with a read by mail, behind all kernels it
@@ -638,8 +649,10 @@ int fsig_match_noalloc(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32
   // event is recorded (profiling off), nothing is allocated on the device
   Arena saved_arena = c->arena;
   unsigned long long* saved_counters = c->d_counters;
+  const bool saved_open = c->counters_open;
   const bool saved_prof = c->profiling;
   c->d_counters = (unsigned long long*)(base + FSIG_NOALLOC_SCRATCH_BYTES);
+  c->counters_open = false;  // cleared below
   c->arena = Arena();
   c->arena.base = base + kScratchOwn;
   c->arena.cap = FSIG_NOALLOC_SCRATCH_BYTES - kScratchOwn;
@@ -661,6 +674,7 @@ int fsig_match_noalloc(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32
   if (rc == FSIG_ENOMEM) c->err = "noalloc: the static scratch is exhausted (" + c->err + ")";
   c->arena = saved_arena;
   c->d_counters = saved_counters;
+  c->counters_open = saved_open;
   c->profiling = saved_prof;
   return rc;
 }

@@ -85,6 +85,9 @@ struct fsig_ctx {
   // kernel family f (word 2f algorithmic bytes, 2f+1 units); see block_add.
   // Host staging is pinned.
   unsigned long long* d_counters = nullptr;
+  // the per-launch results may hold what a call left that did not end well
+  // (see begin_counters)
+  bool counters_open = false;
   // kPinnedWords words of pinned staging, then the mailbox flag: a kernel
   // writes words here and then mail_seq to the flag, and the host polls it
   unsigned long long* h_pinned = nullptr;
@@ -222,6 +225,11 @@ constexpr size_t kCounterWords = 2 * kStripes * kStripeWords;
 inline unsigned long long* family_counters(fsig_ctx* c, int fam) {
   return c->d_counters + kStripes * kStripeWords + 2 * fam;
 }
+// A call that uses the per-launch results begins with begin_counters and, when
+// it ended well, closes them (counters_open = false): each launch's results
+// were then taken, which leaves them zero.  After a call that failed between a
+// launch and its take they are not, and the next begin_counters clears them.
+int begin_counters(fsig_ctx* c);
 // Reads the sums of the first n words of striped counters and zeroes them
 // (so every launch finds its results at zero).
 int take_striped(fsig_ctx* c, unsigned long long* dev, uint64_t* host, uint32_t n);

@@ -1,0 +1,93 @@
+"""A match that fails on its way leaves nothing behind: after an error
+reported at any of its launches, the next match on the same context finds
+what it finds on a fresh one.  The errors come from the host: a small library
+that stands in front of the HIP runtime reports one failed launch, whose
+kernel runs all the same.  It is loaded before the engine, in a process of
+its own."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SHIM = r"""
+#include <dlfcn.h>
+static int (*real)(void);
+static int left = -1;
+int shim_real(const char* path) {
+  void* h = dlopen(path, RTLD_LAZY);
+  real = h ? (int (*)(void))dlsym(h, "hipGetLastError") : 0;
+  return real != 0;
+}
+void shim_arm(int n) { left = n; }
+int shim_left(void) { return left; }
+int hipGetLastError(void) {
+  const int e = real ? real() : 0;
+  return left >= 0 && left-- == 0 ? 719 : e;  /* hipErrorLaunchFailure */
+}
+"""
+
+CHILD = r"""
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+import fsig_amd as F
+ctx = F.Context(0, 1 << 30)
+hip = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+assert shim.shim_real(hip.encode())
+g = F.HostGraph.chung_lu(30000, 120000, 2.4, 3).set_labels("zipf", 4, 1.2, 4)
+dg = ctx.upload(g, pcsr=True)
+star = F.Query(4, [1, 0, 2, 0], [(0, 1), (0, 2), (0, 3)])
+path = F.Query(5, [0, 1, 0, 2, 0], [(i, i + 1) for i in range(4)])
+mix = F.Query(4, [0, 1, 0, 2], [(0, 1), (1, 2), (0, 2), (2, 3)])
+calls = {
+    "tail": lambda: F.match(dg, mix).count,
+    "chain": lambda: F.match(dg, path).count,
+    "product": lambda: F.match(dg, star).count,
+    "levels": lambda: (ctx.set_tune(fused_tail=1), F.match(dg, mix).count, ctx.set_tune())[1],
+    "alg 2": lambda: F.match(dg, mix, F.ALG_GSI).count,
+    "alg 2 leaves": lambda: F.match(dg, path, F.ALG_GSI).count,
+    "digest": lambda: F.match_digest(dg, mix),
+    "bounded batch": lambda: [int(c) for c in F.match_batch(dg, [mix, path], bounds=[10 ** 9] * 2)[0]],
+}
+want = {n: f() for n, f in calls.items()}
+bad, failed = [], 0
+for name, f in calls.items():
+    if name == "bounded batch":  # only as the call after a failed one
+        continue
+    for n in range(200):
+        shim.shim_arm(n)
+        try:
+            got = f()
+            assert got == want[name], (name, n, got, want[name])
+        except F.FsigError as e:
+            assert e.code == F.FSIG_EHIP, (name, n, e)
+            failed += 1
+        ctx.set_tune()
+        reached = shim.shim_left() < 0
+        shim.shim_arm(-1)
+        if not reached:
+            break
+        for after in (name, "bounded batch" if n % 4 == 0 else "tail"):
+            got = calls[after]()
+            if got != want[after]:
+                bad.append((name, n, after, got, want[after]))
+    else:
+        raise AssertionError("the match never got through")
+    print(name, "launch checks:", n, flush=True)
+assert failed > 40, failed
+assert not bad, bad
+print("ok", failed)
+"""
+
+
+def test_next_match_after_a_failed_one(tmp_path):
+    (tmp_path / "shim.c").write_text(SHIM)
+    so = str(tmp_path / "shim.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", so, str(tmp_path / "shim.c"), "-ldl"], check=True)
+    r = subprocess.run([sys.executable, "-u", "-c", CHILD, so], cwd=ROOT, capture_output=True, text=True, timeout=100,
+                       env=dict(os.environ, PYTHONPATH=ROOT))
+    assert r.returncode == 0 and r.stdout.strip().splitlines()[-1].startswith("ok"), r.stdout[-2000:] + r.stderr[-2000:]
