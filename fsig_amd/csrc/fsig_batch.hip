@@ -2309,6 +2309,7 @@ static int batch_impl(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint3
 extern "C" int fsig_match_batch(fsig_ctx* c, const fsig_graph* g, uint32_t nq, const uint32_t* ks,
                                 const int32_t* const* qlabels, const uint32_t* const* qoff,
                                 const uint32_t* const* qadj, uint64_t* counts_out, double* join_ms) {
+  const CtxLock lk(c);
   return batch_impl(c, g, nq, ks, qlabels, qoff, qadj, nullptr, counts_out, nullptr, join_ms);
 }
 
@@ -2316,6 +2317,7 @@ extern "C" int fsig_match_batch_bounded(fsig_ctx* c, const fsig_graph* g, uint32
                                         const int32_t* const* qlabels, const uint32_t* const* qoff,
                                         const uint32_t* const* qadj, const uint64_t* max_embeddings,
                                         uint64_t* counts_out, int32_t* status_out, double* join_ms) {
+  const CtxLock lk(c);
   if (c && !max_embeddings) return set_err(c, FSIG_EINVAL, "batch: null bounds");
   return batch_impl(c, g, nq, ks, qlabels, qoff, qadj, max_embeddings, counts_out, status_out, join_ms);
 }

@@ -581,12 +581,14 @@ extern "C" {
 int fsig_match(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_t* qlabels, const uint32_t* qoff,
                const uint32_t* qadj, const uint32_t* qsig, int alg, int mode, uint64_t max_emb,
                uint64_t* count_out, uint32_t* emb_out, uint64_t emb_cap) {
+  const CtxLock lk(c);
   return match_impl(c, g, k, qlabels, qoff, qadj, qsig, alg, mode, max_emb, count_out, emb_out, emb_cap, nullptr);
 }
 
 int fsig_match_digest(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_t* qlabels, const uint32_t* qoff,
                       const uint32_t* qadj, const uint32_t* qsig, int alg, uint64_t* count_out,
                       uint64_t* digest_out) {
+  const CtxLock lk(c);
   if (c && !digest_out) return set_err(c, FSIG_EINVAL, "digest: null digest");
   return match_impl(c, g, k, qlabels, qoff, qadj, qsig, alg, FSIG_MODE_ENUMERATE, 0, count_out, nullptr, 0,
                     digest_out);
@@ -632,6 +634,7 @@ extern "C" {
 int fsig_match_noalloc(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_t* qlabels, const uint32_t* qoff,
                        const uint32_t* qadj, const uint32_t* qsig, int alg, int mode, uint64_t max_emb,
                        uint64_t* count_out, uint32_t* emb_out, uint64_t emb_cap) {
+  const CtxLock lk(c);
   if (!c) return FSIG_EINVAL;
   if (!g || !count_out) return set_err(c, FSIG_EINVAL, "noalloc: null argument");
   // the candidate mask (4 bytes a vertex) and the candidate arrays (at most
@@ -701,6 +704,7 @@ int fsig_last_candidate_set(const fsig_ctx* c, uint32_t u, int stage, uint32_t* 
 }
 
 int fsig_stream_copy(fsig_ctx* c, uint64_t bytes, uint32_t iters, double* gbps) {
+  const CtxLock lk(c);
   if (!c || !gbps || bytes < 16 || iters == 0) return set_err(c, FSIG_EINVAL, "stream_copy: bad argument");
   FSIG_HIP(c, hipSetDevice(c->device));
   const uint64_t n = bytes / 16;
@@ -738,6 +742,7 @@ int fsig_set_profiling(fsig_ctx* c, int on) {
 }
 
 int fsig_stats_reset(fsig_ctx* c) {
+  const CtxLock lk(c);
   if (!c) return FSIG_EINVAL;
   FSIG_HIP(c, hipSetDevice(c->device));
   const int rc = fetch_stats(c);  // zeroes the device's part
@@ -747,6 +752,7 @@ int fsig_stats_reset(fsig_ctx* c) {
 }
 
 int fsig_kernel_stats(const fsig_ctx* c, int fam, uint64_t* launches, double* ms, uint64_t* bytes, uint64_t* units) {
+  const CtxLock lk(c);
   if (!c || fam < 0 || fam >= FSIG_K_NUM) return FSIG_EINVAL;
   // the device's part of the statistics stays there until somebody asks
   fsig_ctx* m = const_cast<fsig_ctx*>(c);

@@ -132,6 +132,7 @@ extern "C" int fsig_project_bytes(uint32_t n, uint32_t num_labels, const uint64_
 }
 
 extern "C" int fsig_graph_label_pairs(fsig_ctx* c, const fsig_graph* g, uint64_t* pair_edges) {
+  const CtxLock lk(c);
   if (!c) return FSIG_EINVAL;
   if (!g || !pair_edges) return set_err(c, FSIG_EINVAL, "label pairs: null argument");
   if (g->num_labels > kServeMaxLabels) return set_err(c, FSIG_EINVAL, "label pairs: more than 4096 labels");

@@ -6,6 +6,7 @@
 #include <array>
 #include <cstdint>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -62,6 +63,9 @@ struct TimedLaunch {
 };
 
 struct fsig_ctx {
+  // held by every call that uses the stream with the arena, the counters or
+  // the mailbox (CtxLock)
+  mutable std::mutex busy;
   int device = 0;
   hipStream_t stream = nullptr;
   Arena arena;
@@ -175,6 +179,16 @@ void plan_order_mmatch(QueryPlan& P, const uint32_t* class_size);
 bool plan_symmetry(QueryPlan& P);
 void plan_order_gsi(QueryPlan& P, const uint32_t* class_size);
 
+// One such call of a context at a time: the statistics are read by other
+// threads than the one that matches (a monitor), and their fetch takes the
+// mailbox that a running match waits on.
+struct CtxLock {
+  std::unique_lock<std::mutex> lk;
+  explicit CtxLock(const fsig_ctx* c) {
+    if (c) lk = std::unique_lock<std::mutex>(c->busy);
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Error helpers.
 int set_err(fsig_ctx* c, int code, const std::string& msg);
@@ -241,9 +255,8 @@ inline uint32_t refine_passes(const fsig_ctx* c) { return c->tune.refine_passes 
 
 // The context's mailbox: a kernel of its stream writes its words to
 // Mail::words and then, with mail_flag(flag, seq), the flag; mail_wait
-// returns once the flag has arrived.  One mail is on its way at a time (a
-// context is used by one thread at a time) and its words are read before the
-// next is sent.  The kernels before the sender have then finished; later ones
+// returns once the flag has arrived.  One mail is on its way at a time (CtxLock)
+// and its words are read before the next is sent.  The kernels before the sender have then finished; later ones
 // may still run.
 struct Mail {
   unsigned long long* words;

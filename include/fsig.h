@@ -197,7 +197,13 @@ int fsig_last_batch_tune(const fsig_ctx* ctx, uint32_t* lanes_per_row, uint32_t*
 
 /* Per-kernel-family statistics of the context, accumulated since the last
  * fsig_stats_reset.  With profiling on, every launch of the family is
- * bracketed by HIP events on the context stream and its time is summed. */
+ * bracketed by HIP events on the context stream and its time is summed.
+ * Part of them stays on the device until it is asked for: fsig_kernel_stats
+ * and fsig_stats_reset launch a small kernel on the context's stream and wait
+ * for it (FSIG_EHIP when that fails).  Calls of one context that use its
+ * stream run one after another, whatever threads make them: a thread that
+ * reads the statistics of a context whose match is running waits for the
+ * match. */
 enum {
   FSIG_K_FILTER = 0,   /* label/degree or signature filter + compaction  */
   FSIG_K_REFINE = 1,   /* count-based refinement passes                  */
