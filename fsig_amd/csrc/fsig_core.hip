@@ -182,6 +182,7 @@ int scan_u32_to_u64(fsig_ctx* c, const uint32_t* in, uint64_t* out, uint64_t n, 
 
 int resolve_events(fsig_ctx* c) {
   for (size_t i = 0; i < c->timed_used; i++) {
+    if (!c->timed[i].closed) continue;
     float ms = 0;
     FSIG_HIP(c, hipEventElapsedTime(&ms, c->timed[i].a, c->timed[i].b));
     c->kstat[c->timed[i].fam].ms += ms;
@@ -545,12 +546,14 @@ static int match_impl(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
   if (alg == FSIG_ALG_MMATCH) {
     bool by_degree = false;
     for (uint32_t u = 0; u < k; u++) by_degree |= P.aut > 1 && P.sym_adj[u] != 0 && c->work_limit == 0;
-    const size_t mk2 = c->arena.mark(), timed = c->timed_used;
+    const size_t mk2 = c->arena.mark();
+    const std::string err = by_degree ? c->err : std::string();
     rc = run_mmatch(c, g, P, mode, run_bound, count_out, emb_out, emb_cap, acc, by_degree);
-    if (rc == FSIG_ENOMEM && by_degree) {
-      // the two orders build different tables: the arena may hold only the other's
+    if (by_degree && (rc == FSIG_ENOMEM || rc == FSIG_EUNSUPPORTED)) {
+      // the two orders build different tables: the arena (or the row limit of
+      // the candidate edges) may hold only the other's
       c->arena.release(mk2);
-      c->timed_used = timed;
+      c->err = err;
       rc = run_mmatch(c, g, P, mode, run_bound, count_out, emb_out, emb_cap, acc, false);
     }
   } else {

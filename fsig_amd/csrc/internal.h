@@ -60,6 +60,7 @@ struct KStat {
 struct TimedLaunch {
   int fam;
   hipEvent_t a, b;
+  bool closed;  // b is recorded (a match that failed leaves pairs without)
 };
 
 struct fsig_ctx {
@@ -209,13 +210,14 @@ struct KTimer {
   explicit KTimer(fsig_ctx* ctx, int family) : c(ctx), fam(family) {
     if (c->profiling) {
       if (c->timed_used == c->timed.size()) {
-        TimedLaunch t{family, nullptr, nullptr};
+        TimedLaunch t{family, nullptr, nullptr, false};
         (void)hipEventCreate(&t.a);
         (void)hipEventCreate(&t.b);
         c->timed.push_back(t);
       }
       slot = c->timed_used++;
       c->timed[slot].fam = family;
+      c->timed[slot].closed = false;
       (void)hipEventRecord(c->timed[slot].a, c->stream);
     }
   }
@@ -226,7 +228,10 @@ struct KTimer {
     s.launches++;
     s.alg_bytes += alg_bytes;
     s.units += units;
-    if (slot != ~(size_t)0) (void)hipEventRecord(c->timed[slot].b, c->stream);
+    if (slot != ~(size_t)0) {
+      (void)hipEventRecord(c->timed[slot].b, c->stream);
+      c->timed[slot].closed = true;
+    }
   }
 };
 // Adds the recorded event intervals into the context statistics; the stream

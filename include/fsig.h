@@ -203,7 +203,10 @@ int fsig_last_batch_tune(const fsig_ctx* ctx, uint32_t* lanes_per_row, uint32_t*
  * for it (FSIG_EHIP when that fails).  Calls of one context that use its
  * stream run one after another, whatever threads make them: a thread that
  * reads the statistics of a context whose match is running waits for the
- * match. */
+ * match.  They count what ran, also in a match that failed, and in a count
+ * that ran out of arena with the degree-ordered symmetry conditions and was
+ * then run with conditions by vertex id (a count that fits neither way fails
+ * after both). */
 enum {
   FSIG_K_FILTER = 0,   /* label/degree or signature filter + compaction  */
   FSIG_K_REFINE = 1,   /* count-based refinement passes                  */
