@@ -924,6 +924,13 @@ struct PlainShared {
   uint32_t s1[GPB][MAXQ], n1[GPB][MAXQ], cf1[GPB][MAXQ];
 };
 
+// A count pass of 16 lanes with fused tails (a batch tuned to 16 lanes) runs
+// six blocks a compute unit, as its registers allow: its arrays, the sums at
+// its end (last_acc, last_q, block_add) and a 16 KiB tile, in steps of 1,280
+// bytes, six times in 160 KiB.
+constexpr size_t kMultiLds = sizeof(TailShared<16>) + 12 * (FSIG_BLOCK / 16) + 16 * (FSIG_BLOCK / 64) + 16384;
+static_assert(6 * ((kMultiLds + 1279) / 1280 * 1280) <= 160 * 1024, "six blocks of the batch's count pass fit");
+
 template <int G, bool WRITE>
 __global__ void __launch_bounds__(FSIG_BLOCK) k_join_multi(const MLevel* __restrict__ ML,
                                                            const uint64_t* __restrict__ qbase, uint32_t nlive,

@@ -397,9 +397,9 @@ struct TailLds {
   uint32_t* s2;
   uint32_t* n2;
   uint32_t* cf2;
-  uint32_t* slot;  // G words each: children counted by the group, and the
-  uint32_t* cs;    // starts and the scanned lengths of their own lists
-  uint32_t* pre;
+  uint32_t* slot;  // G words each: children counted by the group, and
+  uint32_t* cs;    // (kTailBoth) the starts and the scanned lengths of their
+  uint32_t* pre;   // own lists
   uint32_t* tile;  // tw words
   uint32_t tw;
 };
@@ -799,19 +799,34 @@ constexpr uint32_t kTailMax = 16;
 // instead of 25 KiB, so LDS no longer caps the waves per CU.
 constexpr uint32_t kTailSmall = 8;
 
+// Starts and scanned lengths of the own lists of children counted in groups
+// (kTailBoth); the other kinds have none.
+template <int G, bool HELD>
+struct TailOwnLists {
+  uint32_t cs_[FSIG_BLOCK / G][G], pre_[FSIG_BLOCK / G][G];
+  __device__ uint32_t* cs(uint32_t gw) { return cs_[gw]; }
+  __device__ uint32_t* pre(uint32_t gw) { return pre_[gw]; }
+};
+template <int G>
+struct TailOwnLists<G, false> {
+  __device__ uint32_t* cs(uint32_t) { return nullptr; }
+  __device__ uint32_t* pre(uint32_t) { return nullptr; }
+};
+
 // N1: entries of the level-p arrays (MAXQ when a lockstep launch also keeps
 // its plain rows there; the plain tail's levels are limited to kTailMax
 // backward lists and conflicts: less LDS per group, more groups per CU);
 // N2: entries of the leaf-level arrays.
-template <int G, int N1 = MAXQ, int N2 = kTailMax>
-struct TailShared {
+template <int G, int N1 = MAXQ, int N2 = kTailMax, int KIND = kTailAny>
+struct TailShared : TailOwnLists<G, KIND == kTailBoth> {
   static constexpr int GPB = FSIG_BLOCK / G;
   static constexpr uint32_t kTileWords = 4096 / GPB;  // at most 16 KiB of tiles per block
   uint32_t s1[GPB][N1], n1[GPB][N1], cf1[GPB][N1];
   uint32_t s2[GPB][N2], n2[GPB][N2], cf2[GPB][N2];
-  uint32_t slot[GPB][G], cs[GPB][G], pre[GPB][G];
+  uint32_t slot[GPB][G];
   __device__ TailLds at(uint32_t gw, uint32_t* tile, uint32_t tw) {
-    return TailLds{s1[gw], n1[gw], cf1[gw], s2[gw], n2[gw], cf2[gw], slot[gw], cs[gw], pre[gw], tile + gw * tw, tw};
+    return TailLds{s1[gw], n1[gw], cf1[gw], s2[gw], n2[gw], cf2[gw], slot[gw], this->cs(gw), this->pre(gw),
+                   tile + gw * tw, tw};
   }
 };
 
@@ -835,7 +850,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK)
 k_join_tail(JoinLevel L1, CandEdgeSrc S1, JoinLevel L2, CandEdgeSrc S2, TailIO io) {
   constexpr int GPB = FSIG_BLOCK / G;
   constexpr int NR = (MAXQ + G - 1) / G;
-  __shared__ TailShared<G, N, N> sh;
+  __shared__ TailShared<G, N, N, KIND> sh;
   extern __shared__ uint32_t tail_tile[];
   const uint32_t lane = threadIdx.x & 63u, gl = lane & (G - 1), gw = threadIdx.x / G;
   const uint64_t gmask = (G == 64) ? ~0ull : (((1ull << G) - 1) << (lane - gl));
