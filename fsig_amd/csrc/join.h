@@ -398,8 +398,8 @@ struct TailLds {
   uint32_t* n2;
   uint32_t* cf2;
   uint32_t* slot;  // G words each: children counted by the group, and
-  uint32_t* cs;    // (kTailBoth) the starts and the scanned lengths of their
-  uint32_t* pre;   // own lists
+  uint32_t* cs;    // (kTailBoth) the starts and lengths of their own lists
+  uint32_t* cn;
   uint32_t* tile;  // tw words
   uint32_t tw;
 };
@@ -407,6 +407,18 @@ struct TailLds {
 // Lists of the leaf level: only shared ones (of parent columns), only the
 // child's own, or both.
 enum TailKind : int { kTailAny = -1, kTailShared = 0, kTailOwn = 1, kTailBoth = 2 };
+
+// Longest own list that 8 lanes of a group read through (16 steps); longer
+// ones take the whole group, one after another, each searched for the entries
+// of I or, where that is at most a quarter of the work, read through.  One
+// hub among 64 children otherwise kept the other lanes waiting: the 4-cycle
+// bounded by 1,000 on the 2^20-vertex, 8.75M-edge R-MAT graph took 132 ms in
+// groups, 65 ms one child at a time, and takes 48 ms; triangles there with
+// lists by id 49, 25.6 and 26.5 ms.  (256: 27.1 ms, and 7.2 instead of 6.0
+// with lists by degree, many of which have 256..446 entries; 1,024: the
+// 4-cycle 73 ms.  Reading where it is no more work instead of a quarter: the
+// 4-clique on the 2^18-vertex graph, lists by id, 45.7 ms instead of 39.5.)
+constexpr uint32_t kTailLong = 512;
 
 // Leaves of one parent row; returns this lane's share of the leaf count
 // (sum over the group's lanes = the row's leaves) and sets `children` (group
@@ -693,8 +705,7 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
       lds_wave_sync();
       continue;
     }
-    // The surviving children of this step, one per lane: their own lists,
-    // laid end to end by an exclusive scan of the lengths.
+    // the surviving children of this step, one per lane: their own lists
     if (ok) sh.slot[__popcll(bal & below)] = x;
     lds_wave_sync();
     uint32_t cs = 0, cn = 0;
@@ -703,83 +714,102 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
       cs = S2.off[own][xx];
       cn = S2.off[own][xx + 1] - cs;
     }
-    uint32_t pre = cn;
-#pragma unroll
-    for (int o = 1; o < G; o <<= 1) {
-      const uint32_t t2 = __shfl_up(pre, o, G);
-      if (gl >= (uint32_t)o) pre += t2;
-    }
-    const uint32_t tot = __shfl(pre, G - 1, G);
+    // long lists are set aside and taken by the whole group: by 8 lanes each,
+    // one hub among the children of a step held up the others
+    uint64_t longs = (__ballot(cn > kTailLong) & gmask) >> (threadIdx.x & 63u & ~(uint32_t)(G - 1));
+    if (cn > kTailLong) cn = 0;
+    const uint32_t nshort = nsurv - (uint32_t)__popcll(longs);
     sh.cs[gl] = cs;
-    sh.pre[gl] = pre - cn;
+    sh.cn[gl] = cn;
     lds_wave_sync();
+    uint32_t tot = cn;
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) tot += __shfl_xor(tot, o, G);
     const uint32_t* ol = S2.lst[own];
-    const uint32_t pairs = nsurv * isz, lg = 32 - __builtin_clz((tot / nsurv) | 1);
-    if (gl == 0) lbytes += 8ull * nsurv;
-    if ((uint64_t)tot * (hsize ? 1 : 32 - __builtin_clz(isz)) <= (uint64_t)pairs * lg) {
-      // read the lists through: sub-groups of 8 lanes take every (G/8)th
-      // child, four strides of its list in flight, each entry looked up in I
-      constexpr uint32_t SG = G < 8 ? G : 8, NS = G / SG;
-      const uint32_t sl = gl & (SG - 1);
-      uint32_t j = gl / SG, at = 0, n = 0, xx = 0;
-      const uint32_t* l = ol;
-      bool open = false;  // child j is being read: entries [at, n) of l are left
-      for (;;) {
-        if (!open && j < nsurv) {
-          l = ol + sh.cs[j];
-          n = (j + 1 < (uint32_t)G ? sh.pre[j + 1] : tot) - sh.pre[j];
-          xx = sh.slot[j];
-          at = 0;
-          open = true;
-        }
-        if (!open) break;
-        uint32_t y[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          const uint32_t e = at + u * SG + sl;
-          y[u] = e < n ? l[e] : kNone;
-        }
-        at += 4 * SG;
-        if (at >= n) { open = false; j += NS; }
-        if (g2p | l2p) {  // leaves above (g2p) or below (l2p) the child itself
-#pragma unroll
-          for (int u = 0; u < 4; u++)
-            if ((g2p && y[u] <= xx) || (l2p && y[u] >= xx)) y[u] = kNone;
-        }
-        if (hsize) {
-          uint32_t h[4];
-#pragma unroll
-          for (int u = 0; u < 4; u++) h[u] = (y[u] * 0x9e3779b1u) >> hshift;
-          bool more;
-          do {  // the four chains advance together
-            uint32_t v[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) v[u] = hset[h[u]];
-            more = false;
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-              leaves += v[u] == y[u] && y[u] != kNone;
-              const bool on = v[u] != y[u] && v[u] != kNone && y[u] != kNone;
-              h[u] = (h[u] + 1) & (hsize - 1);
-              if (!on) y[u] = kNone;
-              more |= on;
-            }
-          } while (more);
-        } else {
-#pragma unroll
-          for (int u = 0; u < 4; u++) leaves += y[u] != kNone && sorted_contains(sh.tile, isz, y[u]);
-        }
-      }
-      if (gl == 0) lbytes += 4ull * tot;
-    } else {
-      // search them: one (child, entry of I) pair per lane and step
-      for (uint32_t e = gl; e < pairs; e += G) {
+    const uint32_t probe = hsize ? 1 : 32 - __builtin_clz(isz);  // LDS probes of I for an entry read
+    const uint32_t lg = 32 - __builtin_clz((nshort ? tot / nshort : 0) | 1);
+    const bool read = (uint64_t)tot * probe <= (uint64_t)(nshort * isz) * lg;
+    if (gl == 0) lbytes += 8ull * nsurv + (read ? 4ull * tot : 4ull * nshort * isz * lg);
+    if (!read) {
+      // search the short lists: one (child, entry of I) pair per lane and step
+      for (uint32_t e = gl; e < nsurv * isz; e += G) {
         const uint32_t j = e / isz;
         const uint32_t y = sh.tile[e - j * isz], xx = sh.slot[j];
-        const uint32_t s = sh.cs[j], n = (j + 1 < (uint32_t)G ? sh.pre[j + 1] : tot) - sh.pre[j];
+        leaves += !(g2p && y <= xx) && !(l2p && y >= xx) && sorted_contains(ol + sh.cs[j], sh.cn[j], y);
+      }
+    }
+    for (uint64_t m = longs; m; m &= m - 1) {
+      const uint32_t j = (uint32_t)__builtin_ctzll(m), s = sh.cs[j], xx = sh.slot[j];
+      const uint32_t n = S2.off[own][xx + 1] - s, lgn = 32 - __builtin_clz(n);
+      if (4ull * n * probe <= (uint64_t)isz * lgn) {  // read below
+        if (gl == 0) lbytes += 4ull * n;
+        continue;
+      }
+      longs &= ~(1ull << j);
+      if (gl == 0) lbytes += 4ull * isz * lgn;
+      for (uint32_t e = gl; e < isz; e += G) {
+        const uint32_t y = sh.tile[e];
         leaves += !(g2p && y <= xx) && !(l2p && y >= xx) && sorted_contains(ol + s, n, y);
       }
-      if (gl == 0) lbytes += 4ull * pairs * lg;
+    }
+    // Read lists through, four strides of a list in flight, each entry looked
+    // up in I: sub-groups of 8 lanes take every (G/8)th child's short list,
+    // then all lanes the long ones (each lane on its own: no lane waits).
+    constexpr uint32_t SG = G < 8 ? G : 8, NS = G / SG;
+    uint32_t j = read ? gl / SG : nsurv, at = 0, n = 0, w = SG, xx = 0;
+    const uint32_t* l = ol;
+    for (;;) {
+      if (at >= n) {  // the list is done: the next one
+        uint32_t q;
+        if (j < nsurv) {
+          q = j;
+          n = sh.cn[q];
+          at = gl & (SG - 1);
+          j += NS;
+        } else if (longs) {
+          q = (uint32_t)__builtin_ctzll(longs);
+          longs &= longs - 1;
+          n = S2.off[own][sh.slot[q] + 1] - sh.cs[q];
+          at = gl;
+          w = G;
+        } else {
+          break;
+        }
+        l = ol + sh.cs[q];
+        xx = sh.slot[q];
+      }
+      uint32_t y[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) y[u] = at + u * w < n ? l[at + u * w] : kNone;
+      at += 4 * w;
+      if (g2p | l2p) {  // leaves above (g2p) or below (l2p) the child itself
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if ((g2p && y[u] <= xx) || (l2p && y[u] >= xx)) y[u] = kNone;
+      }
+      if (hsize) {
+        uint32_t h[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) h[u] = (y[u] * 0x9e3779b1u) >> hshift;
+        bool more;
+        do {  // the four chains advance together
+          uint32_t v[4];
+#pragma unroll
+          for (int u = 0; u < 4; u++) v[u] = hset[h[u]];
+          more = false;
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            leaves += v[u] == y[u] && y[u] != kNone;
+            const bool on = v[u] != y[u] && v[u] != kNone && y[u] != kNone;
+            h[u] = (h[u] + 1) & (hsize - 1);
+            if (!on) y[u] = kNone;
+            more |= on;
+          }
+        } while (more);
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; u++) leaves += y[u] != kNone && sorted_contains(sh.tile, isz, y[u]);
+      }
     }
     lds_wave_sync();
   }
@@ -799,18 +829,18 @@ constexpr uint32_t kTailMax = 16;
 // instead of 25 KiB, so LDS no longer caps the waves per CU.
 constexpr uint32_t kTailSmall = 8;
 
-// Starts and scanned lengths of the own lists of children counted in groups
+// Starts and lengths of the own lists of children counted in groups
 // (kTailBoth); the other kinds have none.
 template <int G, bool HELD>
 struct TailOwnLists {
-  uint32_t cs_[FSIG_BLOCK / G][G], pre_[FSIG_BLOCK / G][G];
+  uint32_t cs_[FSIG_BLOCK / G][G], cn_[FSIG_BLOCK / G][G];
   __device__ uint32_t* cs(uint32_t gw) { return cs_[gw]; }
-  __device__ uint32_t* pre(uint32_t gw) { return pre_[gw]; }
+  __device__ uint32_t* cn(uint32_t gw) { return cn_[gw]; }
 };
 template <int G>
 struct TailOwnLists<G, false> {
   __device__ uint32_t* cs(uint32_t) { return nullptr; }
-  __device__ uint32_t* pre(uint32_t) { return nullptr; }
+  __device__ uint32_t* cn(uint32_t) { return nullptr; }
 };
 
 // N1: entries of the level-p arrays (MAXQ when a lockstep launch also keeps
@@ -825,7 +855,7 @@ struct TailShared : TailOwnLists<G, KIND == kTailBoth> {
   uint32_t s2[GPB][N2], n2[GPB][N2], cf2[GPB][N2];
   uint32_t slot[GPB][G];
   __device__ TailLds at(uint32_t gw, uint32_t* tile, uint32_t tw) {
-    return TailLds{s1[gw], n1[gw], cf1[gw], s2[gw], n2[gw], cf2[gw], slot[gw], this->cs(gw), this->pre(gw),
+    return TailLds{s1[gw], n1[gw], cf1[gw], s2[gw], n2[gw], cf2[gw], slot[gw], this->cs(gw), this->cn(gw),
                    tile + gw * tw, tw};
   }
 };
@@ -840,13 +870,21 @@ struct TailIO {
   uint32_t kids_are_shared;   // the child level intersects the leaf's shared lists
 };
 
-// N: entries of the per-group list and conflict arrays of both levels.  At
-// most 72 VGPRs, so seven waves per SIMD fit where LDS allows (the tail is
-// bound by dependent gathers; eight waves need spills and run slower); 64
-// four-lane groups with 16-entry arrays fit six per SIMD by their LDS.
+// Waves per SIMD asked of the tail.  It is bound by dependent gathers: seven
+// (72 VGPRs) where LDS allows, as eight need spills and run slower.  Five
+// blocks of four-lane groups with 16-entry arrays fit a compute unit's LDS.
+// Children counted in groups by 16 or 32 lanes spill 5..10 VGPRs at seven and
+// run as fast or faster at six (the 4-clique on the 2^18-vertex R-MAT graph:
+// 6.4 ms against 6.6).
 template <int G, int N, int KIND>
-__global__ void __launch_bounds__(FSIG_BLOCK)
-    __attribute__((amdgpu_waves_per_eu(G == 4 && N > (int)kTailSmall ? 5 : 7, 8)))
+constexpr int tail_waves() {
+  if (G == 4 && N > (int)kTailSmall) return 5;
+  return KIND == kTailBoth && (G == 16 || G == 32) ? 6 : 7;
+}
+
+// N: entries of the per-group list and conflict arrays of both levels.
+template <int G, int N, int KIND>
+__global__ void __launch_bounds__(FSIG_BLOCK) __attribute__((amdgpu_waves_per_eu(tail_waves<G, N, KIND>(), 8)))
 k_join_tail(JoinLevel L1, CandEdgeSrc S1, JoinLevel L2, CandEdgeSrc S2, TailIO io) {
   constexpr int GPB = FSIG_BLOCK / G;
   constexpr int NR = (MAXQ + G - 1) / G;
