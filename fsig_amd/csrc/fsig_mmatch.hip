@@ -161,13 +161,33 @@ __global__ void k_scatter_pos(const uint32_t* __restrict__ cand, uint32_t n, uin
 }
 
 // out[i] = first list entry of pair i; out[np] = the number of list entries,
-// out[np + 1] = *entries: all that the host waits for, in one read.
+// out[np + 1] = *entries, out[np + 2] = 0 (k_longest_oriented): all that the
+// host waits for, in one read.
 __global__ void k_pair_bases(const uint64_t* __restrict__ gscan, const PairDesc* __restrict__ P, uint32_t np,
                              uint64_t rows, const uint64_t* __restrict__ entries, uint64_t* __restrict__ out) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < np) out[i] = gscan[P[i].flat];
   else if (i == np) out[i] = gscan[rows];
   else if (i == np + 1) out[i] = *entries;
+  else if (i == np + 2) out[i] = 0;
+}
+
+// *longest = max(*longest, entries of the longest list ordered by degree).
+__global__ void __launch_bounds__(FSIG_BLOCK) k_longest_oriented(const PairDesc* __restrict__ P, uint32_t np,
+                                                                 uint64_t rows, const uint32_t* __restrict__ cnt,
+                                                                 unsigned long long* __restrict__ longest) {
+  uint32_t m = 0;
+  for (uint64_t f = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; f < rows; f += (uint64_t)gridDim.x * blockDim.x)
+    if (cedge_pair(P, np, f).orient) m = max(m, cnt[f]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor(m, o));
+  __shared__ uint32_t part[FSIG_BLOCK / 64];
+  if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < FSIG_BLOCK / 64; w++) m = max(m, part[w]);
+    if (m) atomicMax(longest, (unsigned long long)m);
+  }
 }
 
 }  // namespace
@@ -186,6 +206,7 @@ struct MMatchProvider {
   // symmetry conditions kept by oriented lists: adj_lt[u] has bit w when
   // phi(u) comes before phi(w) by degree, for neighbours u and w
   uint32_t adj_lt[MAXQ];
+  uint32_t longest;  // bound on the entries of a list ordered by degree (once the lists are built)
 
   // orientation of the list that extends u's image by its neighbour w
   uint32_t orient(uint32_t u, uint32_t w) const {
@@ -204,7 +225,7 @@ struct MMatchProvider {
       const uint32_t u = P->order[c];
       if ((P->adjm[w] >> u) & 1u) {
         L.bcol[L.nb++] = c;
-        if (orient(u, w)) L.oriented = 1;
+        if (orient(u, w)) L.oriented = std::max(longest, 1u);
       } else if (P->label[u] == P->label[w]) {
         const uint32_t j = L.ncf++;
         L.cfcol[j] = c;
@@ -510,7 +531,7 @@ int run_mmatch(fsig_ctx* c, const fsig_graph* g, QueryPlan& P, int mode, uint64_
     PairDesc* dP = (PairDesc*)A.alloc(sizeof(PairDesc) * np);
     uint32_t* cnt = (uint32_t*)A.alloc(4ull * flat);
     uint64_t* gscan = (uint64_t*)A.alloc(8ull * (flat + 1));
-    uint64_t* pbase = (uint64_t*)A.alloc(8ull * (np + 2));
+    uint64_t* pbase = (uint64_t*)A.alloc(8ull * (np + 3));
     if (!dP || !cnt || !gscan || !pbase) return set_err(c, FSIG_ENOMEM, "cedge: arena exhausted");
     FSIG_HIP(c, hipMemcpyAsync(dP, pairs.data(), sizeof(PairDesc) * np, hipMemcpyHostToDevice, c->stream));
     if ((rc = row_count(c, RG, dP, np, flat, g->d_off, g->d_adj, cnt))) return rc;
@@ -519,10 +540,21 @@ int run_mmatch(fsig_ctx* c, const fsig_graph* g, QueryPlan& P, int mode, uint64_
     if ((rc = seg_count(c, dP, np, flat, g->d_off, g->d_adj, cnt, segs))) return rc;
     FSIG_HIP(c, hipGetLastError());
     if ((rc = scan_u32_to_u64(c, cnt, gscan, flat))) return rc;
-    k_pair_bases<<<(np + 2 + 255) / 256, 256, 0, c->stream>>>(gscan, dP, np, flat, segs.segbase + flat + 1, pbase);
+    k_pair_bases<<<(np + 3 + 255) / 256, 256, 0, c->stream>>>(gscan, dP, np, flat, segs.segbase + flat + 1, pbase);
+    // the tail's lanes depend on the longest list ordered by degree; it is
+    // looked for where the largest degree does not settle them
+    bool by_longest = false;
+    if (by_degree && k >= 3) {
+      const JoinLevel Lw = pv.level(k - 1);
+      by_longest = Lw.oriented && Lw.nb == 2;
+    }
+    if (by_longest && g->max_degree > kTailShortLists)
+      k_longest_oriented<<<(uint32_t)std::min<uint64_t>((flat + 4 * FSIG_BLOCK - 1) / (4 * FSIG_BLOCK), c->num_cus),
+                           FSIG_BLOCK, 0, c->stream>>>(dP, np, flat, cnt, (unsigned long long*)pbase + np + 2);
     FSIG_HIP(c, hipGetLastError());
-    std::vector<uint64_t> hb(np + 2);
-    if ((rc = read_u64(c, pbase, hb.data(), np + 2))) return rc;
+    std::vector<uint64_t> hb(np + 3);
+    if ((rc = read_u64(c, pbase, hb.data(), np + 3))) return rc;
+    pv.longest = hb[np + 2] ? (uint32_t)hb[np + 2] : g->max_degree;
     const uint64_t total_edges = hb[np];
     segs.entries = hb[np + 1];
     uint32_t* lst_all = (uint32_t*)A.alloc(4ull * std::max<uint64_t>(total_edges, 1));

@@ -49,9 +49,10 @@ struct JoinLevel {
   // every column in gtmask and stay below that of every column in ltmask
   // (columns of w's class: the words compare as the data vertex ids do)
   uint32_t gtmask, ltmask;
-  uint32_t oriented;  // some list keeps a symmetry condition itself (ordered by degree)
+  // some list keeps a symmetry condition itself (ordered by degree): a bound on
+  // the entries of such lists; else 0
+  uint32_t oriented;
 };
-
 
 constexpr uint32_t kNone = 0xffffffffu;
 
@@ -996,6 +997,16 @@ inline bool tail_kids_shared(const JoinLevel& L1, const CandEdgeSrc& S1, const J
   return j == L1.nb;
 }
 
+// A leaf of one shared and one own list (the triangle), ordered by degree,
+// takes 64 lanes a row and with them the widest tile where some of these lists
+// have more entries than this: few rows then hold most of the work.  8 / 64
+// lanes, by the longest list: 454 entries (2^20-vertex R-MAT graph, average 8)
+// 28.9 / 5.9 ms, 53 (dblp-law graph, 3) 0.70 / 0.58, 21 (1M-vertex Chung-Lu
+// graph, 5) 1.46 / 1.76, 10 (4M-vertex random graph, 4) 4.1 / 5.4, 3 (2,000 x
+// 2,000 triangulated grid) 1.6 / 3.6.  With two shared lists (the 4-clique) rows are
+// many and I is short; the lanes of a mean list do.
+constexpr uint32_t kTailShortLists = 24;
+
 // Tile words per group the tail of L2 needs: only a leaf with both shared
 // lists (parent columns) and an own list (column p) intersects in LDS.
 // 16 KiB per block; 22 KiB where lists ordered by degree are intersected: a
@@ -1490,10 +1501,9 @@ class JoinDriver {
     // through the LDS tile, else few (rows are mostly a handful of dependent
     // gathers: more of them in flight)
     const bool needs_tile = tail_tile_words(8, L2, 0) != 0;
-    // (64 for lists ordered by degree: the widest tile, which holds all of
-    // them with their hash sets)
+    const bool wide = L2.oriented > kTailShortLists && L2.nb == 2 && !c_->tune.lanes_per_row;
     const uint32_t G0 = use_chain || !needs_tile ? std::min<uint32_t>(std::max<uint32_t>(G_, 4), 8)
-                        : L2.oriented && L2.nb == 2 && !c_->tune.lanes_per_row ? 64u : std::max<uint32_t>(G_, 8);
+                        : wide ? 64u : std::max<uint32_t>(G_, 8);
     const uint32_t G = widen_lanes(c_, G0, R, use_chain ? 32 : 64);
     const TailIO io{rows, R, cnt, res, family_counters(c_, FSIG_K_JOIN_TAIL),
                     use_chain ? 0u : tail_tile_words(G, L2, c_->tune.lds_tile),

@@ -54,3 +54,19 @@ def test_four_cycles(gpu_ctx, a, b):
         got = counts(dg, q)
         dg.free()
         assert all(v == want for v in got.values()), (order, want, got)
+
+
+@pytest.mark.parametrize("n,hub", [(4, 0), (24, 0), (25, 0), (26, 0), (25, 40), (26, 40), (3, 40), (120, 700)])
+def test_longest_list_by_degree(gpu_ctx, n, hub):
+    """K_n (its longest list by degree has n - 1 entries) beside a star whose
+    centre's degree says nothing of its lists, on the edge of the rule for the
+    tail's lanes; two triangles that share a vertex have a third list by id."""
+    e = list(itertools.combinations(range(n), 2)) + [(n, n + 1 + i) for i in range(hub)]
+    dg = gpu_ctx.upload(F.HostGraph.from_edges(n + 1 + hub, np.asarray(e, np.uint32)))
+    tri = F.Query(3, np.zeros(3, np.int32), [(0, 1), (1, 2), (0, 2)])
+    bowtie = F.Query(5, np.zeros(5, np.int32), [(0, 1), (1, 2), (0, 2), (2, 3), (3, 4), (2, 4)])
+    got = [counts(dg, q) for q in (tri, bowtie)]
+    dg.free()
+    want = [n * (n - 1) * (n - 2), n * (n - 1) * (n - 2) * (n - 3) * (n - 4)]
+    for g, w in zip(got, want):
+        assert all(v == w for v in g.values()), (w, g)
