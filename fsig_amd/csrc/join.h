@@ -1009,7 +1009,7 @@ constexpr uint32_t kTailShortLists = 24;
 
 // Tile words per group the tail of L2 needs: only a leaf with both shared
 // lists (parent columns) and an own list (column p) intersects in LDS.
-// 16 KiB per block; 22 KiB where lists ordered by degree are intersected: a
+// 16 KiB per block; 22 KiB where long lists ordered by degree are intersected: a
 // wavefront's 1,408 words hold up to 384 entries beside their hash set (the
 // longest list has 446 on the 2^20-vertex R-MAT graph; longer ones are
 // searched), and six blocks fit a compute unit where 32 KiB let four.
@@ -1019,7 +1019,7 @@ inline uint32_t tail_tile_words(uint32_t G, const JoinLevel& L2, uint32_t cap) {
   bool shared = false, own = false;
   for (uint32_t i = 0; i < L2.nb; i++) (L2.bcol[i] == L2.p - 1 ? own : shared) = true;
   if (!shared || !own) return 0;
-  const uint32_t w = (L2.oriented ? 5632 : 4096) / (FSIG_BLOCK / G);
+  const uint32_t w = (L2.oriented > kTailShortLists ? 5632 : 4096) / (FSIG_BLOCK / G);
   return cap && cap < w ? cap : w;
 }
 
