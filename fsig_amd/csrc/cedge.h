@@ -17,6 +17,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "device.h"
 #include "internal.h"
@@ -26,25 +27,47 @@ namespace {
 constexpr uint32_t kHubDeg = 512;
 constexpr uint32_t kSegEdges = 512;
 
-// Whether data vertex x is a candidate of the pair's target class.
-template <class PT>
-__device__ __forceinline__ bool cedge_keep(const PT& pd, uint32_t x) {
-  return pd.bits ? (pd.bits[x >> 5] >> (x & 31u)) & 1u : (pd.mask[x] >> pd.bbit) & 1u;
-}
+// What the entries of one row (the neighbours of candidate v, which has dv of
+// them) are tested with.
+struct CedgeTest {
+  const uint32_t* bits;  // candidates of the target class: their bitmap, or (null)
+  const uint32_t* mask;  // bit bbit of a word per vertex
+  const uint32_t* off;
+  uint32_t bbit, orient, v, dv;
+};
 
-// cedge_keep for neighbour x of v (degree dv), and in an oriented pair also
-// the order of the two: by degree, then id, x past v (orient 1) or before it
-// (orient 2).  The degree order keeps the lists of a power-law graph short:
-// the longest list towards higher degrees has 446 entries on the 2^20-vertex,
-// 8.75M-edge R-MAT graph, where ids leave half of the 42,300 neighbours.
-template <class PT>
-__device__ __forceinline__ bool cedge_keep(const PT& pd, const uint32_t* __restrict__ off, uint32_t v, uint32_t dv,
-                                           uint32_t x) {
-  if (!cedge_keep(pd, x)) return false;
-  if (!pd.orient) return true;
-  const uint32_t dx = off[x + 1] - off[x];
-  const bool past = dx != dv ? dx > dv : x > v;
-  return past == (pd.orient == 1);
+// ok[t] &= whether x[t] (0 where ok[t] is false) is a candidate of the target
+// class and, in an oriented pair, past v (orient 1) or before it (orient 2)
+// by degree, then id.  The degree order keeps the lists of a power-law graph
+// short: the longest list towards higher degrees has 454 entries on the
+// 2^20-vertex, 8.75M-edge R-MAT graph, where ids leave half of the 42,300
+// neighbours.  Its price is a gather per entry and pass, so all entries' words
+// are loaded before any is looked at: the build of the diamond's lists there
+// went from 0.91 to 0.71 ms (one entry after another before; 0.61 without an
+// order), the bowtie's from 1.33 to 1.02.
+template <int U>
+__device__ __forceinline__ void cedge_keep(const CedgeTest& T, const uint32_t (&x)[U], bool (&ok)[U]) {
+  uint32_t w[U];
+  uint2 o[U];
+  if (T.bits) {
+#pragma unroll
+    for (int t = 0; t < U; t++) w[t] = T.bits[x[t] >> 5] >> (x[t] & 31u);
+  } else {
+#pragma unroll
+    for (int t = 0; t < U; t++) w[t] = T.mask[x[t]] >> T.bbit;
+  }
+  if (T.orient) {
+#pragma unroll
+    for (int t = 0; t < U; t++) __builtin_memcpy(&o[t], T.off + x[t], 8);  // both offsets in one load
+#pragma unroll
+    for (int t = 0; t < U; t++) {
+      const uint32_t dx = o[t].y - o[t].x;
+      const bool past = dx != T.dv ? dx > T.dv : x[t] > T.v;
+      ok[t] = ok[t] && past == (T.orient == 1);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < U; t++) ok[t] = ok[t] && (w[t] & 1u);
 }
 
 // Pair of flat row f: the last pair whose first row is <= f.
@@ -144,12 +167,28 @@ __device__ __forceinline__ XcdRange xcd_range(uint64_t n, uint32_t per_block, ui
 // loaded before any is tested, so a group keeps U gathers in flight.
 constexpr int kRowUnroll = 4;
 
+// Calls body(U, j) for the strides of a row's entries [s, e): kRowUnroll at a
+// time while some group of the wavefront has more than one left, else one (on
+// a graph of 6 neighbours a vertex, three of four strides would be empty).
+template <int G, class Body>
+__device__ __forceinline__ void row_strides(uint32_t s, uint32_t e, const Body& body) {
+  for (uint32_t j = s; j < e;) {
+    if (__ballot(e - j > (uint32_t)G)) {
+      body(std::integral_constant<int, kRowUnroll>(), j);
+      j += kRowUnroll * G;
+    } else {
+      body(std::integral_constant<int, 1>(), j);
+      j += G;
+    }
+  }
+}
+
 template <class PT, int G>
 __global__ void __launch_bounds__(FSIG_BLOCK) k_row_count(const PT* __restrict__ P, uint32_t np, uint64_t rows,
                                                           const uint32_t* __restrict__ off,
                                                           const uint32_t* __restrict__ adj,
                                                           uint32_t* __restrict__ cnt) {
-  constexpr int GPB = FSIG_BLOCK / G, U = kRowUnroll;
+  constexpr int GPB = FSIG_BLOCK / G;
   const uint32_t lane = threadIdx.x & 63u, gl = lane & (G - 1), gw = threadIdx.x / G;
   const uint64_t gmask = (G == 64) ? ~0ull : (((1ull << G) - 1) << (lane - gl));
   const XcdRange xr = xcd_range(rows, GPB, gw);
@@ -158,8 +197,10 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_row_count(const PT* __restrict__
     const uint32_t v = pd.acand[f - pd.flat];
     const uint32_t s = off[v], e = off[v + 1];
     if (e - s > kHubDeg) continue;  // k_seg_cedge
+    const CedgeTest T{pd.bits, pd.mask, off, pd.bbit, pd.orient, v, e - s};
     uint32_t got = 0;
-    for (uint32_t j = s; j < e; j += U * G) {
+    row_strides<G>(s, e, [&](auto un, uint32_t j) {
+      constexpr int U = decltype(un)::value;
       uint32_t x[U];
       bool ok[U];
 #pragma unroll
@@ -168,11 +209,10 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_row_count(const PT* __restrict__
         ok[t] = i < e;
         x[t] = ok[t] ? adj[i] : 0u;
       }
-#pragma unroll
-      for (int t = 0; t < U; t++) ok[t] = ok[t] && cedge_keep(pd, off, v, e - s, x[t]);
+      cedge_keep(T, x, ok);
 #pragma unroll
       for (int t = 0; t < U; t++) got += (uint32_t)__popcll(__ballot(ok[t]) & gmask);
-    }
+    });
     if (gl == 0) cnt[f] = got;
   }
 }
@@ -183,7 +223,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_row_fill(const PT* __restrict__ 
                                                          const uint32_t* __restrict__ adj,
                                                          const uint64_t* __restrict__ gscan,
                                                          uint32_t* __restrict__ lst_all) {
-  constexpr int GPB = FSIG_BLOCK / G, U = kRowUnroll;
+  constexpr int GPB = FSIG_BLOCK / G;
   const uint32_t lane = threadIdx.x & 63u, gl = lane & (G - 1), gw = threadIdx.x / G;
   const uint64_t gmask = (G == 64) ? ~0ull : (((1ull << G) - 1) << (lane - gl));
   const uint64_t below = (1ull << lane) - 1;
@@ -194,13 +234,18 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_row_fill(const PT* __restrict__ 
     const uint32_t v = pd.acand[i0];
     const uint32_t s = off[v], e = off[v + 1];
     if (e - s > kHubDeg) continue;  // k_seg_cedge
-    const uint64_t pbase = gscan[pd.flat];
+    const uint64_t pbase = gscan[pd.flat], to = gscan[f + 1];
     uint64_t at = gscan[f];
     if (gl == 0) {
       pd.off_out[i0] = (uint32_t)(at - pbase);
-      if (i0 + 1 == pd.asize) pd.off_out[pd.asize] = (uint32_t)(gscan[f + 1] - pbase);
+      if (i0 + 1 == pd.asize) pd.off_out[pd.asize] = (uint32_t)(to - pbase);
     }
-    for (uint32_t j = s; j < e; j += U * G) {
+    if (to == at) continue;                // no entry kept
+    const bool all = to - at == e - s;     // every entry kept: no second test
+    const CedgeTest T{pd.bits, pd.mask, off, pd.bbit, pd.orient, v, e - s};
+    const uint32_t* bpos = pd.bpos;
+    row_strides<G>(s, e, [&](auto un, uint32_t j) {
+      constexpr int U = decltype(un)::value;
       uint32_t x[U];
       bool ok[U];
 #pragma unroll
@@ -209,15 +254,14 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_row_fill(const PT* __restrict__ 
         ok[t] = i < e;
         x[t] = ok[t] ? adj[i] : 0u;
       }
-#pragma unroll
-      for (int t = 0; t < U; t++) ok[t] = ok[t] && cedge_keep(pd, off, v, e - s, x[t]);
+      if (!all) cedge_keep(T, x, ok);
 #pragma unroll
       for (int t = 0; t < U; t++) {
         const uint64_t bal = __ballot(ok[t]) & gmask;
-        if (ok[t]) lst_all[at + __popcll(bal & below)] = pd.bpos ? pd.bpos[x[t]] : sorted_index(pd.bcand, pd.bsize, x[t]);
+        if (ok[t]) lst_all[at + __popcll(bal & below)] = bpos ? bpos[x[t]] : sorted_index(pd.bcand, pd.bsize, x[t]);
         at += __popcll(bal);
       }
-    }
+    });
   }
 }
 
@@ -269,8 +313,7 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_seg_cedge(const PT* __restrict__
         ok[t] = i < s1;
         x[t] = ok[t] ? adj[i] : 0u;
       }
-#pragma unroll
-      for (int t = 0; t < 8; t++) ok[t] = ok[t] && cedge_keep(pd, off, v, dv, x[t]);
+      cedge_keep(CedgeTest{pd.bits, pd.mask, off, pd.bbit, pd.orient, v, dv}, x, ok);
       uint32_t got = 0;
       unsigned long long mine = 0;
 #pragma unroll

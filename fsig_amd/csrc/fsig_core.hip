@@ -544,8 +544,9 @@ static int match_impl(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
   if (mode == FSIG_MODE_COUNT && !digest_out && c->tune.symmetry == 0 && plan_symmetry(P) && P.aut > 1 && max_emb)
     run_bound = max_emb / P.aut + (max_emb % P.aut != 0);
   if (alg == FSIG_ALG_MMATCH) {
+    // (an edge alone is not intersected with anything)
     bool by_degree = false;
-    for (uint32_t u = 0; u < k; u++) by_degree |= P.aut > 1 && P.sym_adj[u] != 0 && c->work_limit == 0;
+    for (uint32_t u = 0; u < k; u++) by_degree |= k > 2 && P.aut > 1 && P.sym_adj[u] != 0 && c->work_limit == 0;
     const size_t mk2 = c->arena.mark();
     const std::string err = by_degree ? c->err : std::string();
     rc = run_mmatch(c, g, P, mode, run_bound, count_out, emb_out, emb_cap, acc, by_degree);
