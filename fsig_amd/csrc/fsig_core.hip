@@ -601,15 +601,17 @@ int fsig_match_digest(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32_
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
-// Static scratch of fsig_match_noalloc: the device counters (first 512
-// bytes) and the arena of one match.  Each device that loads the library
-// holds its own copy until the process ends.  In host code `scratch` names a
+// Static scratch of fsig_match_noalloc: the arena of one match, then its
+// counters.  Each device that loads the library holds its own copy until the
+// process ends.  In host code `scratch` names a
 // host-side stand-in, never the device memory: its device address is taken
 // once per device with hipGetSymbolAddress and only that address is used.
-// Of the promised bytes, 512 are the engine's own; its counters follow the
-// array's end.
-constexpr size_t kScratchOwn = 512;
-static __device__ __align__(256) char scratch[FSIG_NOALLOC_SCRATCH_BYTES + kCounterWords * sizeof(unsigned long long)];
+// (The arena is 512 bytes short of the stated size, the counters' place when
+// they were fewer: the graphs that fit stay the same.)
+constexpr size_t kScratchArena = FSIG_NOALLOC_SCRATCH_BYTES - 512;
+static __device__ __align__(256) char scratch[kScratchArena + kCounterWords * sizeof(unsigned long long)];
+static_assert(sizeof(scratch) == FSIG_NOALLOC_SCRATCH_BYTES + 7680, "the size that fsig.h states");
+static_assert(kScratchArena % sizeof(unsigned long long) == 0, "the counters are aligned");
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -644,7 +646,7 @@ int fsig_match_noalloc(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32
   // the candidate mask (4 bytes a vertex) and the candidate arrays (at most
   // 4 bytes a vertex of the query's labels, twice) must fit with room left
   const uint64_t need = 12ull * g->n + (1u << 20);
-  if (need > FSIG_NOALLOC_SCRATCH_BYTES - kScratchOwn)
+  if (need > kScratchArena)
     return set_err(c, FSIG_EINVAL,
                    "noalloc: a graph of " + std::to_string(g->n) + " vertices needs at least " +
                        std::to_string(need) + " bytes of scratch, more than the static " +
@@ -658,11 +660,11 @@ int fsig_match_noalloc(fsig_ctx* c, const fsig_graph* g, uint32_t k, const int32
   unsigned long long* saved_counters = c->d_counters;
   const bool saved_open = c->counters_open;
   const bool saved_prof = c->profiling;
-  c->d_counters = (unsigned long long*)(base + FSIG_NOALLOC_SCRATCH_BYTES);
+  c->d_counters = (unsigned long long*)(base + kScratchArena);
   c->counters_open = false;  // cleared below
   c->arena = Arena();
-  c->arena.base = base + kScratchOwn;
-  c->arena.cap = FSIG_NOALLOC_SCRATCH_BYTES - kScratchOwn;
+  c->arena.base = base;
+  c->arena.cap = kScratchArena;
   c->profiling = false;
   rc = FSIG_OK;
   // the counters must start at zero: earlier calls leave theirs behind

@@ -92,6 +92,10 @@ void fsig_graph_free(fsig_ctx* ctx, fsig_graph* g);
  *        FSIG_MODE_ENUMERATE: embeddings are materialised in HBM; the first
  *        min(count, emb_cap) rows are copied to emb_out (host, k words per
  *        row, query-vertex order) when emb_out != NULL.
+ *        A count returns when its result has arrived in pinned host memory;
+ *        a last kernel that does not touch it, the graph or the query may
+ *        still be on the context's stream (fsig_ctx_synchronize waits for it,
+ *        and later calls of the context run behind it).
  *   max_embeddings (0 = no bound) bounds both modes: the work stops once
  *        that many embeddings are found and *count_out = min(count,
  *        max_embeddings); pass L+1 to ask "more than L?".  Which embeddings
@@ -119,14 +123,16 @@ int fsig_match_digest(fsig_ctx* ctx, const fsig_graph* g, uint32_t k, const int3
 
 /* fsig_match for callers that cannot allocate device memory (tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the
- * reference.  The match synchronises its stream between levels, so the call
- * cannot itself be captured into a HIP graph.  Same arguments, results
- * and errors as fsig_match, but every buffer of the match beyond its inputs
- * and outputs (candidate masks and arrays, candidate-edge lists, join
- * tables, scan partials, counters, the staging of emb_out) comes from one
- * static device array of FSIG_NOALLOC_SCRATCH_BYTES, which each GPU that
- * loads the library holds until the process ends; the call allocates no
- * device memory and records no profiling events.  The graph and the
+ * reference.  The match waits between levels for totals that its kernels
+ * write to pinned host memory, so the call cannot itself be captured into a
+ * HIP graph.  Same arguments, results and errors as fsig_match, but every
+ * buffer of the match beyond its inputs and outputs (candidate masks and
+ * arrays, candidate-edge lists, join tables, scan partials, counters, the
+ * staging of emb_out) comes from one static device array of
+ * FSIG_NOALLOC_SCRATCH_BYTES and 7,680 bytes (the tables, then the
+ * counters), which each GPU that loads the library holds until the process
+ * ends; the call allocates no device memory, records no profiling events and
+ * returns when its kernels are done with the array.  The graph and the
  * context's stream and pinned host staging are the caller's, made before.
  * A graph too large for the scratch is rejected with FSIG_EINVAL (at least
  * 12 bytes a vertex plus 1 MiB must fit); a match that runs out of scratch
