@@ -313,7 +313,18 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_seg_cedge(const PT* __restrict__
         ok[t] = i < s1;
         x[t] = ok[t] ? adj[i] : 0u;
       }
-      cedge_keep(CedgeTest{pd.bits, pd.mask, off, pd.bbit, pd.orient, v, dv}, x, ok);
+      if (pd.orient) {
+        cedge_keep(CedgeTest{pd.bits, pd.mask, off, pd.bbit, pd.orient, v, dv}, x, ok);
+      } else {
+        // one stride after another: with all eight in flight the bitmap's
+        // lines come from beyond L2 more often (529 -> 728 MB a launch on the
+        // 16M-vertex graph), which one match alone hides (its pass takes 2.0
+        // instead of 2.1 ms) and six workers do not (32 served requests
+        // 142.0 instead of 141.1 ms)
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+          ok[t] = ok[t] && ((pd.bits ? pd.bits[x[t] >> 5] >> (x[t] & 31u) : pd.mask[x[t]] >> pd.bbit) & 1u);
+      }
       uint32_t got = 0;
       unsigned long long mine = 0;
 #pragma unroll
