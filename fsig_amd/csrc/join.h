@@ -409,8 +409,8 @@ struct TailLds {
 // child's own, or both.
 enum TailKind : int { kTailAny = -1, kTailShared = 0, kTailOwn = 1, kTailBoth = 2 };
 
-// Longest own list that 8 lanes of a group read through (16 steps); longer
-// ones take the whole group, one after another, each searched for the entries
+// Longest own list that 8 of a group's 16 or more lanes read through (16
+// steps); longer ones take the whole group, one after another, each searched for the entries
 // of I or, where that is at most a quarter of the work, read through.  One
 // hub among 64 children otherwise kept the other lanes waiting: the 4-cycle
 // bounded by 1,000 on the 2^20-vertex, 8.75M-edge R-MAT graph took 132 ms in
@@ -611,18 +611,24 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
       return 0;
     }
   }
-  // I as an open-addressing hash set behind its list in the tile, a quarter
-  // to half full, when several children will be intersected with it: a child's
-  // list is then read through once, in coalesced steps, and each entry costs
-  // about two LDS reads instead of a chain of dependent gathers.  Bound by
-  // the latency of those reads and of the row's own range lookups.  With
-  // lists ordered by degree, the triangle on the 2^20-vertex, 8.75M-edge
-  // R-MAT graph went from 27.7 to 7.1 ms and the 4-clique on the 2^18-vertex,
-  // 2.19M-edge one from 37.6 to 8.0 ms (6.0 and 6.2 ms now; one child at a
-  // time and binary searches, ordered by degree: 17.5 and 11.8 ms).
+  // I as an open-addressing hash set behind its list in the tile, an eighth
+  // to a quarter full (up to half where the tile holds no more), when several
+  // children will be intersected with it: a child's list is then read through
+  // once, in coalesced steps, and each entry costs about two LDS reads instead
+  // of a chain of dependent gathers.  Bound by vector instructions (issued in
+  // 44 % of the cycles in the triangle's tail, 69 % in the 4-clique's) and the
+  // waits for lists and LDS between them.  With lists ordered by degree, the
+  // triangle on the 2^20-vertex, 8.75M-edge R-MAT graph went from 27.7 to 7.1
+  // ms and the 4-clique on the 2^18-vertex, 2.19M-edge one from 37.6 to 8.0 ms
+  // (5.9 and 6.3 ms now; one child at a time and binary searches, ordered by
+  // degree: 17.5 and 11.8 ms).  Lists by id are often too long to read and are
+  // searched, and groups of 8 and 16 lanes then build a set per row for
+  // nothing: a 14-path and one edge on the labeled 1M-vertex graph took 366 ms
+  // without sets, 1,015 with, and takes 375 ms (from 32 lanes the 4-cycle of
+  // kTailLong takes 48 ms with sets, 62 without).
   uint32_t hsize = 0, hshift = 0;
   uint32_t* hset = sh.tile + isz;
-  if (KIND == kTailBoth && !defer_row && 2 * isz > (uint32_t)G && tb1 - ta1 > 2) {
+  if (KIND == kTailBoth && (G >= 32 || L2.oriented) && !defer_row && 2 * isz > (uint32_t)G && tb1 - ta1 > 2) {
     hshift = __builtin_clz(2 * isz - 1) - 1;
     if (isz + (1u << (32 - hshift)) > sh.tw) hshift++;
     hsize = 1u << (32 - hshift);
@@ -717,8 +723,8 @@ __device__ __forceinline__ uint64_t tail_row(const JoinLevel& L1, const CandEdge
     }
     // long lists are set aside and taken by the whole group: by 8 lanes each,
     // one hub among the children of a step held up the others
-    uint64_t longs = (__ballot(cn > kTailLong) & gmask) >> (threadIdx.x & 63u & ~(uint32_t)(G - 1));
-    if (cn > kTailLong) cn = 0;
+    uint64_t longs = (__ballot(G > 8 && cn > kTailLong) & gmask) >> (threadIdx.x & 63u & ~(uint32_t)(G - 1));
+    if (G > 8 && cn > kTailLong) cn = 0;
     const uint32_t nshort = nsurv - (uint32_t)__popcll(longs);
     sh.cs[gl] = cs;
     sh.cn[gl] = cn;
