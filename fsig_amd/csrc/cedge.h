@@ -39,11 +39,11 @@ struct CedgeTest {
 // ok[t] &= whether x[t] (0 where ok[t] is false) is a candidate of the target
 // class and, in an oriented pair, past v (orient 1) or before it (orient 2)
 // by degree, then id.  The degree order keeps the lists of a power-law graph
-// short: the longest list towards higher degrees has 454 entries on the
+// short: the longest list towards higher degrees has some 450 entries on the
 // 2^20-vertex, 8.75M-edge R-MAT graph, where ids leave half of the 42,300
 // neighbours.  Its price is a gather per entry and pass, so all entries' words
 // are loaded before any is looked at: the build of the diamond's lists there
-// went from 0.91 to 0.71 ms (one entry after another before; 0.61 without an
+// went from 0.91 to 0.71 ms (one entry after another before; 0.48 without an
 // order), the bowtie's from 1.33 to 1.02.
 template <int U>
 __device__ __forceinline__ void cedge_keep(const CedgeTest& T, const uint32_t (&x)[U], bool (&ok)[U]) {
@@ -109,8 +109,9 @@ __global__ void __launch_bounds__(FSIG_BLOCK) k_seg_rows(const PT* __restrict__ 
     if (hub) cnt[f] = 0;
     mine += deg;
   }
-  // one addition per block, and few blocks: additions to one word take 12 ns
-  // each (80 us of a 2^20-row launch when every wavefront made one)
+  // one addition per block, and few blocks: additions to one word go one
+  // after another (the launch over the 2^20-vertex R-MAT graph's candidates
+  // took 80 us when every wavefront with a row made one, 15 now)
   __shared__ uint64_t lds[4];
   mine = block_sum(mine, lds);
   if (threadIdx.x == 0 && mine) atomicAdd(entries, mine);

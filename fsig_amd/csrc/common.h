@@ -133,8 +133,8 @@ __global__ void k_emit(EmitMap M, const uint32_t* __restrict__ rows, uint64_t n,
 
 // Digest of level-k rows: one row per thread, words taken in query-vertex
 // order; per-wave sums are added to M.acc[0..1].  A match's last level is
-// digested as it is found (k_join); this takes tables that are there already
-// (a query of one vertex, a bounded match).
+// digested as it is found (k_join); this takes the table of a query of one
+// vertex.
 __global__ void __launch_bounds__(FSIG_BLOCK) k_digest(DigestMap M, const uint32_t* __restrict__ rows, uint64_t n) {
   unsigned long long s0 = 0, s1 = 0;
   for (uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += (uint64_t)gridDim.x * blockDim.x) {

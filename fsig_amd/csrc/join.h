@@ -416,7 +416,7 @@ enum TailKind : int { kTailAny = -1, kTailShared = 0, kTailOwn = 1, kTailBoth = 
 // bounded by 1,000 on the 2^20-vertex, 8.75M-edge R-MAT graph took 132 ms in
 // groups, 65 ms one child at a time, and takes 48 ms; triangles there with
 // lists by id 49, 25.6 and 26.5 ms.  (256: 27.1 ms, and 7.2 instead of 6.0
-// with lists by degree, many of which have 256..446 entries; 1,024: the
+// with lists by degree, many of which have 256..450 entries; 1,024: the
 // 4-cycle 73 ms.  Reading where it is no more work instead of a quarter: the
 // 4-clique on the 2^18-vertex graph, lists by id, 45.7 ms instead of 39.5.)
 constexpr uint32_t kTailLong = 512;
@@ -945,9 +945,10 @@ __device__ __forceinline__ uint32_t list_less_conflicts(const JoinLevel& L, cons
 // one parent column, so a row's leaves are the product of two list lengths,
 // less conflicts.  One lane per row: it is a chain of a dozen dependent
 // gathers with nothing to share, bound by how many rows are in flight, and a
-// group of lanes repeats the same gathers.  The 8-path on the 317,080-vertex
-// dblp-law graph: 2.0 ms in this tail with four lanes a row, 1.9 ms for the
-// whole match now (2.5 and 3.9 ms for two seeds before).
+// group of lanes repeats the same gathers.  The tail of the 8-path on a
+// 317,080-vertex dblp-law graph: 4.1 ms with four lanes a row (and statistics
+// added by every wavefront), 1.2 ms here; on the benchmark's graph 0.55 ms at
+// 1.3 TB/s of memory traffic, most of its gathers hitting L2.
 static __global__ void __launch_bounds__(FSIG_BLOCK) k_join_tail_product(JoinLevel L1, CandEdgeSrc S1, JoinLevel L2,
                                                                   CandEdgeSrc S2, TailIO io) {
   unsigned long long leaves = 0, kids = 0, bytes = 0, rows = 0;
@@ -1006,18 +1007,18 @@ inline bool tail_kids_shared(const JoinLevel& L1, const CandEdgeSrc& S1, const J
 // A leaf of one shared and one own list (the triangle), ordered by degree,
 // takes 64 lanes a row and with them the widest tile where some of these lists
 // have more entries than this: few rows then hold most of the work.  8 / 64
-// lanes, by the longest list: 454 entries (2^20-vertex R-MAT graph, average 8)
-// 28.9 / 5.9 ms, 53 (dblp-law graph, 3) 0.70 / 0.58, 21 (1M-vertex Chung-Lu
-// graph, 5) 1.46 / 1.76, 10 (4M-vertex random graph, 4) 4.1 / 5.4, 3 (2,000 x
-// 2,000 triangulated grid) 1.6 / 3.6.  With two shared lists (the 4-clique) rows are
-// many and I is short; the lanes of a mean list do.
+// lanes, by the longest list: some 450 entries (2^20-vertex R-MAT graph,
+// average 8) 28.9 / 5.9 ms, 53 (dblp-law graph, 3) 0.70 / 0.58, 21 (1M-vertex
+// Chung-Lu graph, 5) 1.46 / 1.76, 10 (4M-vertex random graph, 4) 4.1 / 5.4, 3
+// (2,000 x 2,000 triangulated grid) 1.6 / 3.6.  With two shared lists (the
+// 4-clique) rows are many and I is short: the lanes of a mean list do.
 constexpr uint32_t kTailShortLists = 24;
 
 // Tile words per group the tail of L2 needs: only a leaf with both shared
 // lists (parent columns) and an own list (column p) intersects in LDS.
 // 16 KiB per block; 22 KiB where long lists ordered by degree are intersected: a
 // wavefront's 1,408 words hold up to 384 entries beside their hash set (the
-// longest list has 446 on the 2^20-vertex R-MAT graph; longer ones are
+// longest list has some 450 on the 2^20-vertex R-MAT graph; longer ones are
 // searched), and six blocks fit a compute unit where 32 KiB let four.
 // Triangle on that graph / 4-clique on the 2^18-vertex one: 32 KiB 7.1 / 6.9
 // ms, 24 KiB 6.3 / 6.2, 22 KiB 6.0 / 6.2, 20 KiB 7.0 / 5.7, 16 KiB 7.4 / 6.0.
@@ -1242,10 +1243,15 @@ static __global__ void k_window_rows(const uint64_t* __restrict__ off, uint64_t 
                                      unsigned long long* __restrict__ out) {
   const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
   // Entries [0, a) lie below the answer, entry b (if there is one) does not.
-  // The last entries of `parts` parts lie below it, so a moves past those
-  // parts, and stays at most b: the next part ends at na + step - 1 >= na.
-  // (Taking the smaller of the two instead of na itself was compiled to a
-  // select on the comparison before it.)
+  // [a, b) is cut into parts of `step` entries, one a lane; the parts whose
+  // last entry lies below the answer are counted by the ballot, and a moves
+  // past them.  It needs no bound: the next part ends at a + step - 1 >= a,
+  // and so does the new b.  Bounding it all the same, by b and in front of the
+  // select for b, has been compiled to two scalar selects on one condition,
+  // the first one's: a became b where it had to stay below it, the next step
+  // was 0, and rows outside the table were taken.  Two 64-bit minima of
+  // wave-uniform values in a row are read in the assembly before they are
+  // relied on here; the write pass bounds the range it is given.
   uint64_t a = 0, b = nrows + 1;
   while (a < b) {
     const uint64_t step = (b - a + 63) / 64;
