@@ -88,6 +88,5 @@ def test_next_match_after_a_failed_one(tmp_path):
     (tmp_path / "shim.c").write_text(SHIM)
     so = str(tmp_path / "shim.so")
     subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", so, str(tmp_path / "shim.c"), "-ldl"], check=True)
-    r = subprocess.run([sys.executable, "-u", "-c", CHILD, so], cwd=ROOT, capture_output=True, text=True, timeout=100,
-                       env=dict(os.environ, PYTHONPATH=ROOT))
+    r = subprocess.run([sys.executable, "-u", "-c", CHILD, so], cwd=ROOT, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and r.stdout.strip().splitlines()[-1].startswith("ok"), r.stdout[-2000:] + r.stderr[-2000:]
